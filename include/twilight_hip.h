@@ -836,6 +836,19 @@ int tw_rms_norm_gemv_rope(const void* h_in, const void* delta, const void* norm_
 int tw_rms_norm_gemv_silu(const void* h_in, const void* delta, const void* norm_weight, float eps, void* h_out,
                           const void* W, const void* bias, void* y, int N, int K, int dtype, void* stream);
 
+/* ------------------------------------------------------------------------
+ * Dense causal attention of a prompt: out[s][head] = softmax over rows
+ * t <= s of (q . k_t * softmax_scale) times v_t, fp32 accumulation -- the
+ * attention of the reference's prefill (mp.py:475-482).  q row s of head h
+ * (h = g * R + r) is at q + s * q_row + h * q_head, k and v rows of KV head g
+ * likewise (strides in elements, multiples of 8; 16-byte aligned bases); out
+ * is [S][G * R][D] contiguous.  fp16 / bf16, D = 128, softmax_scale > 0,
+ * S <= 2^24; anything else returns TW_EUNSUPPORTED.
+ * ---------------------------------------------------------------------- */
+int tw_prefill_attention(const void* q, const void* k, const void* v, int dtype, int S, int G, int R, int D,
+                         int64_t q_row, int64_t q_head, int64_t k_row, int64_t k_head, int64_t v_row,
+                         int64_t v_head, float softmax_scale, void* out, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

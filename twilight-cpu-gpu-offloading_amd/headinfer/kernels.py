@@ -1804,6 +1804,38 @@ def decode_attention_varlen(
     return out
 
 
+# ----------------------------------------------------------------- prefill
+def prefill_attention_fits(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: float) -> bool:
+    """Whether prefill_attention takes these operands: 16-bit device tensors of one device with head_dim 128, rows
+    of contiguous channels that start on 16 bytes, and a positive scale."""
+    if q.ndim != 4 or k.ndim != 4 or v.shape != k.shape or q.shape[0] != 1 or k.shape[0] != 1:
+        return False
+    if q.dtype not in (torch.float16, torch.bfloat16) or k.dtype != q.dtype or v.dtype != q.dtype:
+        return False
+    if not (q.is_cuda and k.device == q.device and v.device == q.device):
+        return False
+    _, Hq, S, D = q.shape
+    if D != 128 or k.shape[2:] != (S, D) or not 0 < S <= 1 << 24 or k.shape[1] == 0 or Hq % k.shape[1] or Hq == 0:
+        return False
+    return scale > 0.0 and all(t.stride(3) == 1 and t.stride(1) % 8 == 0 and t.stride(2) % 8 == 0
+                               and t.data_ptr() % 16 == 0 for t in (q, k, v))
+
+
+def prefill_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: float) -> torch.Tensor:
+    """Dense causal attention of a prompt (mp.py:475-482) in one launch: q [1, Hq, S, 128] and k/v [1, G, S, 128],
+    any strides prefill_attention_fits takes -> [1, S, Hq*128]."""
+    if not prefill_attention_fits(q, k, v, scale):
+        raise ValueError("prefill_attention takes 16-bit [1, H, S, 128] device tensors with 16-byte aligned rows")
+    _, Hq, S, D = q.shape
+    G = k.shape[1]
+    out = torch.empty((1, S, Hq * D), dtype=q.dtype, device=q.device)
+    with on_device(q.device):
+        check(hip().tw_prefill_attention(ptr(q), ptr(k), ptr(v), _dt(q), S, G, Hq // G, D, q.stride(2), q.stride(1),
+                                         k.stride(2), k.stride(1), v.stride(2), v.stride(1), float(scale), ptr(out),
+                                         stream_handle(q.device)), "prefill_attention")
+    return out
+
+
 # ------------------------------------------------------------ row movement
 _DEVICE_ALIAS: dict[int, int] = {}
 

@@ -36,6 +36,7 @@ import types
 from typing import Any, Optional
 
 import torch
+from torch.autograd import forward_ad
 
 from . import kernels
 
@@ -78,12 +79,23 @@ def _flash_attention_varlen_forward(
 
 
 # ------------------------------------------------------------------ prefill
+def _derivative_wanted(*tensors: torch.Tensor) -> bool:
+    """Whether autograd follows these tensors, backward or forward: the HIP kernels record no derivative."""
+    if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
+        return True
+    return forward_ad._current_level >= 0 and any(forward_ad.unpack_dual(t).tangent is not None for t in tensors)
+
+
 def _prefill_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: float,
                        chunk: int = 1024) -> torch.Tensor:
     """Dense causal attention of a prompt, q [1, Hq, S, D], k/v [1, G, S, D]
-    -> [1, S, Hq*D].  Query chunks keep the score tile bounded; the key
-    operand is materialised transposed and contiguous, scores and softmax in
-    fp32, p.v with p in the input dtype."""
+    -> [1, S, Hq*D].  The matrix-core kernel takes what it can run (16-bit,
+    head_dim 128) when no derivative is asked for; otherwise torch products
+    over query chunks that keep the score tile bounded: the key operand is
+    materialised transposed and contiguous, scores and softmax in fp32, p.v
+    with p in the input dtype."""
+    if not _derivative_wanted(q, k, v) and kernels.prefill_attention_fits(q, k, v, scale):
+        return kernels.prefill_attention(q, k, v, scale)
     _, Hq, S, D = q.shape
     G = k.shape[1]
     R = Hq // G
