@@ -842,12 +842,33 @@ int tw_rms_norm_gemv_silu(const void* h_in, const void* delta, const void* norm_
  * attention of the reference's prefill (mp.py:475-482).  q row s of head h
  * (h = g * R + r) is at q + s * q_row + h * q_head, k and v rows of KV head g
  * likewise (strides in elements, multiples of 8; 16-byte aligned bases); out
- * is [S][G * R][D] contiguous.  fp16 / bf16, D = 128, softmax_scale > 0,
+ * is [S][G * R][D] contiguous.  With cos / sin (both or neither), q is rotated
+ * on the way in as x * cos + rotate_half(x) * sin, each product and the sum
+ * rounded to the storage type, by their row s (at s * cos_row, s * sin_row;
+ * k as given).  fp16 / bf16, D = 128, softmax_scale > 0,
  * S <= 2^24; anything else returns TW_EUNSUPPORTED.
  * ---------------------------------------------------------------------- */
 int tw_prefill_attention(const void* q, const void* k, const void* v, int dtype, int S, int G, int R, int D,
                          int64_t q_row, int64_t q_head, int64_t k_row, int64_t k_head, int64_t v_row,
-                         int64_t v_head, float softmax_scale, void* out, void* stream);
+                         int64_t v_head, const void* cos, const void* sin, int64_t cos_row, int64_t sin_row,
+                         float softmax_scale, void* out, void* stream);
+
+/* ------------------------------------------------------------------------
+ * A prompt's K and V of one layer into the cache (the prefill write and
+ * metadata of quest_offload_cache.py:230-289, twilight_offload_cache.py:
+ * 925-936) with K's rotary embedding before them: row t of KV head g, at
+ * k + t * k_row + g * k_head (v likewise), K rotated by row t of cos / sin as
+ * above, goes to out_k / out_v + g * out_entry_stride + t * D; the rotated
+ * rows' page min/max and, unless packed is null, INT4 codes as
+ * tw_build_page_metadata gives them for entry g.  Strides in elements (rows
+ * for quant_entry_stride); every 16-bit row 16-byte aligned.  fp16 / bf16,
+ * D = 128, 16-row pages, T <= 2^24; anything else returns TW_EUNSUPPORTED.
+ * ---------------------------------------------------------------------- */
+int tw_prompt_kv(const void* k, const void* v, int64_t k_row, int64_t k_head, int64_t v_row, int64_t v_head,
+                 const void* cos, const void* sin, int64_t cos_row, int64_t sin_row, int dtype, int T, int G, int D,
+                 int sink, int block_size, void* out_k, void* out_v, int64_t out_entry_stride, void* page_min,
+                 void* page_max, int64_t page_entry_stride, void* packed, void* scale, void* minimum,
+                 int64_t quant_entry_stride, void* stream);
 
 #ifdef __cplusplus
 }

@@ -29,6 +29,7 @@
 // SIMD, whose products run under the first one's exponentials, is worth more.
 #pragma clang fp contract(off)
 
+#include "rope.h"
 #include "tw_common.h"
 
 namespace tw {
@@ -51,6 +52,9 @@ struct PrefillArgs {
   const uint16_t* v;
   uint16_t* out;
   int64_t q_row, q_head, k_row, k_head, v_row, v_head, out_row;  // in elements
+  const uint16_t* cos;  // nullable: q is rotated by row s of cos / sin as it is loaded
+  const uint16_t* sin;
+  int64_t cos_row, sin_row;
   int S, G, R, tiles;
   float scale_log2;
 };
@@ -118,6 +122,28 @@ __global__ __launch_bounds__(NW * kWave, 2) void prefill_attn_kernel(PrefillArgs
   const uint16_t* qp = a.q + head * a.q_head + static_cast<int64_t>(row < S ? row : S - 1) * a.q_row + 8 * half;
 #pragma unroll
   for (int s = 0; s < 8; ++s) qf[s] = __builtin_bit_cast(frag, *reinterpret_cast<const u32x4*>(qp + 16 * s));
+  if (a.cos != nullptr) {
+    // a rotation pair is 64 channels apart: fragments s and s + 4 of the lane
+    const int64_t at = row < S ? row : S - 1;
+    const uint16_t* cp = a.cos + at * a.cos_row + 8 * half;
+    const uint16_t* sp = a.sin + at * a.sin_row + 8 * half;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const u32x4 x = __builtin_bit_cast(u32x4, qf[s]), y = __builtin_bit_cast(u32x4, qf[s + 4]);
+      const u32x4 cx = *reinterpret_cast<const u32x4*>(cp + 16 * s);
+      const u32x4 cy = *reinterpret_cast<const u32x4*>(cp + 16 * s + 64);
+      const u32x4 sx = *reinterpret_cast<const u32x4*>(sp + 16 * s);
+      const u32x4 sy = *reinterpret_cast<const u32x4*>(sp + 16 * s + 64);
+      u32x4 rx, ry;
+#pragma unroll
+      for (int p = 0; p < 4; ++p) {
+        rx[p] = rope_word<DT>(x[p], y[p] ^ 0x80008000u, cx[p], sx[p]);
+        ry[p] = rope_word<DT>(y[p], x[p], cy[p], sy[p]);
+      }
+      qf[s] = __builtin_bit_cast(frag, rx);
+      qf[s + 4] = __builtin_bit_cast(frag, ry);
+    }
+  }
 
   const int last_row = q_block + NW * kQ - 1;
   const int n_keys = (last_row < S ? last_row : S - 1) + 1;
@@ -272,7 +298,8 @@ int launch_any(const PrefillArgs& a, hipStream_t s) {
 
 extern "C" int tw_prefill_attention(const void* q, const void* k, const void* v, int dtype, int S, int G, int R, int D,
                                     int64_t q_row, int64_t q_head, int64_t k_row, int64_t k_head, int64_t v_row,
-                                    int64_t v_head, float softmax_scale, void* out, void* stream) {
+                                    int64_t v_head, const void* cos, const void* sin, int64_t cos_row, int64_t sin_row,
+                                    float softmax_scale, void* out, void* stream) {
   using namespace tw;
   if (S < 0 || G <= 0 || R <= 0) return TW_EINVAL;
   if (S == 0) return TW_OK;
@@ -280,11 +307,12 @@ extern "C" int tw_prefill_attention(const void* q, const void* k, const void* v,
   if (D != kHead || (dtype != TW_DTYPE_F16 && dtype != TW_DTYPE_BF16) || !(softmax_scale > 0.0f))
     return TW_EUNSUPPORTED;
   if (static_cast<int64_t>((S + 127) / 128) * G * R > 0x7fffffff || S > (1 << 24)) return TW_EUNSUPPORTED;
-  const int64_t strides[] = {q_row, q_head, k_row, k_head, v_row, v_head};
+  if ((cos == nullptr) != (sin == nullptr)) return TW_EINVAL;
+  const int64_t strides[] = {q_row, q_head, k_row, k_head, v_row, v_head, cos_row, sin_row};
   for (const int64_t s : strides)
     if (s < 0 || s % 8 != 0) return TW_EINVAL;  // every row starts on 16 bytes
   if (((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) | reinterpret_cast<uintptr_t>(v) |
-        reinterpret_cast<uintptr_t>(out)) & 15) != 0)
+        reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(cos) | reinterpret_cast<uintptr_t>(sin)) & 15) != 0)
     return TW_EINVAL;
   PrefillArgs a;
   a.q = static_cast<const uint16_t*>(q);
@@ -292,6 +320,8 @@ extern "C" int tw_prefill_attention(const void* q, const void* k, const void* v,
   a.v = static_cast<const uint16_t*>(v);
   a.out = static_cast<uint16_t*>(out);
   a.q_row = q_row, a.q_head = q_head, a.k_row = k_row, a.k_head = k_head, a.v_row = v_row, a.v_head = v_head;
+  a.cos = static_cast<const uint16_t*>(cos), a.sin = static_cast<const uint16_t*>(sin);
+  a.cos_row = cos_row, a.sin_row = sin_row;
   a.out_row = static_cast<int64_t>(G) * R * D;
   a.S = S, a.G = G, a.R = R;
   a.scale_log2 = softmax_scale * 1.4426950408889634f;

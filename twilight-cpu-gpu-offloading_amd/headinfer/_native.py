@@ -124,7 +124,10 @@ _HIP_SIGNATURES = {
     "tw_gather_heads": (i32, [vp, vp, i64, i64, i64, vp, i32, i32, i32, i32, i32, i32, i32, vp, vp, i32, i32, i64,
                               i64, i64, i64, vp, vp, vp, vp]),
     "tw_host_device_pointer": (i32, [vp, ctypes.POINTER(ctypes.c_void_p)]),
-    "tw_prefill_attention": (i32, [vp, vp, vp, i32, i32, i32, i32, i32, i64, i64, i64, i64, i64, i64, f32, vp, vp]),
+    "tw_prefill_attention": (i32, [vp, vp, vp, i32, i32, i32, i32, i32, i64, i64, i64, i64, i64, i64, vp, vp, i64, i64,
+                                   f32, vp, vp]),
+    "tw_prompt_kv": (i32, [vp, vp, i64, i64, i64, i64, vp, vp, i64, i64, i32, i32, i32, i32, i32, i32, vp, vp, i64, vp,
+                           vp, i64, vp, vp, vp, i64, vp]),
     "tw_append_kv": (i32, [vp, vp, i32, i32, i32, vp, vp, i64, i32, i64, vp]),
 }
 

@@ -1821,19 +1821,83 @@ def prefill_attention_fits(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, sc
                                and t.data_ptr() % 16 == 0 for t in (q, k, v))
 
 
-def prefill_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: float) -> torch.Tensor:
+def rope_tables_fit(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> bool:
+    """Whether the prompt kernels can rotate x [1, H, S, 128] by cos/sin: [1, S, 128] tables of x's type and device,
+    rows of contiguous channels that start on 16 bytes."""
+    return all(t.shape == (1, x.shape[2], x.shape[3]) and t.dtype == x.dtype and t.device == x.device
+               and t.stride(2) == 1 and t.stride(1) % 8 == 0 and t.data_ptr() % 16 == 0 for t in (cos, sin))
+
+
+def prefill_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: float,
+                      rope: Optional[tuple[torch.Tensor, torch.Tensor]] = None) -> torch.Tensor:
     """Dense causal attention of a prompt (mp.py:475-482) in one launch: q [1, Hq, S, 128] and k/v [1, G, S, 128],
-    any strides prefill_attention_fits takes -> [1, S, Hq*128]."""
+    any strides prefill_attention_fits takes -> [1, S, Hq*128].  rope: (cos, sin) tables that rotate q (not k) on the
+    way in, as rope_tables_fit takes them."""
     if not prefill_attention_fits(q, k, v, scale):
         raise ValueError("prefill_attention takes 16-bit [1, H, S, 128] device tensors with 16-byte aligned rows")
+    if rope is not None and not rope_tables_fit(q, *rope):
+        raise ValueError("prefill_attention takes [1, S, 128] cos/sin tables of q's type with 16-byte aligned rows")
     _, Hq, S, D = q.shape
     G = k.shape[1]
+    cos, sin = (None, None) if rope is None else rope
     out = torch.empty((1, S, Hq * D), dtype=q.dtype, device=q.device)
     with on_device(q.device):
         check(hip().tw_prefill_attention(ptr(q), ptr(k), ptr(v), _dt(q), S, G, Hq // G, D, q.stride(2), q.stride(1),
-                                         k.stride(2), k.stride(1), v.stride(2), v.stride(1), float(scale), ptr(out),
-                                         stream_handle(q.device)), "prefill_attention")
+                                         k.stride(2), k.stride(1), v.stride(2), v.stride(1), ptr(cos), ptr(sin),
+                                         0 if cos is None else cos.stride(1), 0 if sin is None else sin.stride(1),
+                                         float(scale), ptr(out), stream_handle(q.device)), "prefill_attention")
     return out
+
+
+def prompt_kv(k: torch.Tensor, v: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, out_k: torch.Tensor,
+              out_v: torch.Tensor, *, sink: int, block_size: int, page_min: Optional[torch.Tensor] = None,
+              page_max: Optional[torch.Tensor] = None, packed: Optional[torch.Tensor] = None,
+              scale: Optional[torch.Tensor] = None, minimum: Optional[torch.Tensor] = None) -> None:
+    """A prompt's K/V [1, G, S, 128] (K before its rotary embedding) into rows [0, S) of out_k/out_v [G, >=S, 128], with
+    the rotated keys' page min/max [G, >=P, 128] and, if given, INT4 keys (packed [G, >=S, 64], scale/minimum
+    [G, >=S]), in one launch."""
+    dev = _require_device(k, v, cos, sin, out_k, out_v, page_min, page_max, packed, scale, minimum, what="prompt_kv")
+    _, G, S, D = k.shape
+    pages = (S - sink) // block_size if S > sink else 0
+    if D != 128 or block_size != 16 or k.dtype not in (torch.float16, torch.bfloat16):
+        raise ValueError("prompt_kv takes 16-bit keys of 128 channels and 16-row pages")
+    if v.shape != k.shape or v.dtype != k.dtype or k.shape[0] != 1 or not rope_tables_fit(k, cos, sin):
+        raise ValueError("prompt_kv takes K/V [1, G, S, 128] and [1, S, 128] tables of one type")
+    if any(t.stride(3) != 1 or t.stride(1) % 8 or t.stride(2) % 8 or t.data_ptr() % 16 for t in (k, v)):
+        raise ValueError("K/V rows must be contiguous and start on 16 bytes")
+    for t in (out_k, out_v):
+        if t.dtype != k.dtype or t.ndim != 3 or t.shape[0] != G or t.shape[1] < S or t.shape[2] != D:
+            raise ValueError("prompt_kv destinations are [G, >=S, 128] of the key type")
+    if out_k.stride(2) != 1 or out_k.stride(1) != D or out_v.stride() != out_k.stride():
+        raise ValueError("prompt_kv destination rows must be contiguous")
+    pe = 0
+    if pages:
+        if page_min is None or page_max is None:
+            raise ValueError("prompt_kv needs page_min and page_max")
+        for t in (page_min, page_max):
+            if t.dtype != k.dtype or t.ndim != 3 or t.shape[0] != G or t.shape[1] < pages or t.shape[2] != D:
+                raise ValueError("page metadata buffers are too small")
+        if page_min.stride(2) != 1 or page_min.stride(1) != D or page_max.stride() != page_min.stride():
+            raise ValueError("page metadata buffers must be row-contiguous")
+        pe = page_min.stride(0)
+    qe = 0
+    if packed is not None:
+        if scale is None or minimum is None or scale.dtype != k.dtype or minimum.dtype != k.dtype:
+            raise ValueError("INT4 outputs must be given together in the key dtype")
+        if packed.dtype != torch.uint8 or packed.ndim != 3 or packed.shape[0] != G or packed.shape[1] < S \
+                or packed.shape[2] != D // 2 or packed.stride(2) != 1 or packed.stride(1) != D // 2 \
+                or packed.stride(0) % (D // 2):
+            raise ValueError("packed buffer has the wrong shape")
+        qe = packed.stride(0) // (D // 2)
+        for t in (scale, minimum):
+            if t.shape[0] != G or t.shape[1] < S or t.stride(1) != 1 or t.stride(0) != qe:
+                raise ValueError("scale/minimum must share the packed entry stride")
+    with on_device(dev):
+        check(hip().tw_prompt_kv(ptr(k), ptr(v), k.stride(2), k.stride(1), v.stride(2), v.stride(1), ptr(cos), ptr(sin),
+                                 cos.stride(1), sin.stride(1), _dt(k), S, G, D, sink, block_size, ptr(out_k),
+                                 ptr(out_v), out_k.stride(0), ptr(page_min) if pages else None,
+                                 ptr(page_max) if pages else None, pe, ptr(packed), ptr(scale), ptr(minimum), qe,
+                                 stream_handle(dev)), "prompt_kv")
 
 
 # ------------------------------------------------------------ row movement

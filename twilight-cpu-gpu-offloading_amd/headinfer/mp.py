@@ -178,6 +178,15 @@ def _decode(self, cache, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> t
     return torch.cat(outs).reshape(1, 1, Hq * D)
 
 
+def _fused_prompt(cache: Any, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: torch.Tensor,
+                  sin: torch.Tensor, scale: float) -> bool:
+    """Whether a prompt takes the two-launch path (K/V rotation, cache write and metadata; attention that rotates q):
+    nothing asks for a derivative and every operand is of the form those kernels read."""
+    return (_is_headinfer_cache(cache) and hasattr(cache, "prompt_layer_fits")
+            and not _derivative_wanted(q, k, v, cos, sin) and kernels.prefill_attention_fits(q, k, v, scale)
+            and kernels.rope_tables_fit(q, cos, sin) and cache.prompt_layer_fits(k, v, cos, sin))
+
+
 def _fast_forward(self, hidden_states: torch.Tensor, position_embeddings=None, attention_mask=None,
                   past_key_values=None, **kwargs):
     from transformers.models.llama.modeling_llama import apply_rotary_pos_emb
@@ -190,8 +199,12 @@ def _fast_forward(self, hidden_states: torch.Tensor, position_embeddings=None, a
     k = self.k_proj(hidden_states).view(hidden_shape).transpose(1, 2)
     v = self.v_proj(hidden_states).view(hidden_shape).transpose(1, 2)
     cos, sin = position_embeddings
-    q, k = apply_rotary_pos_emb(q, k, cos, sin)
     cache = past_key_values
+    if q_len > 1 and _fused_prompt(cache, q, k, v, cos, sin, float(self.scaling)):
+        keys, values = cache.update_prompt_layer(self._headinfer_entry0, k, v, cos, sin)
+        attn = kernels.prefill_attention(q, keys, values, float(self.scaling), rope=(cos, sin))
+        return self.o_proj(attn), None
+    q, k = apply_rotary_pos_emb(q, k, cos, sin)
     if not _is_headinfer_cache(cache):
         raise ValueError("a headinfer-patched model needs a QuestTopKOffloadedCache / "
                          "TwilightMatchedBudgetOffloadedCache as past_key_values")

@@ -56,6 +56,10 @@ class _CacheBase(_HFCache):  # type: ignore[misc, valid-type]
             super().__init__()
 
 
+# The per-entry prompt methods that update_prompt_layer stands in for.
+_PROMPT_HOOKS = frozenset({"update", "_build_metadata", "_write_prompt"})
+
+
 def _window(length: int, sink: int, recent: int) -> tuple[int, int, int]:
     """(sink_end, recent_start, eligible) of quest_offload_cache.py:326-333."""
     sink_end = min(sink, length)
@@ -323,18 +327,76 @@ class QuestTopKOffloadedCache(_CacheBase):
         }
 
     # ---------------------------------------------------------------- prefill
-    def _build_metadata(self, entry: int, key_states: torch.Tensor) -> None:
-        """Page min/max of the prompt's complete pages (quest_offload_cache.py:276-289)."""
-        keys = key_states[0, 0]
-        T = int(keys.shape[0])
+    def _allocate_metadata(self, T: int) -> int:
+        """The metadata buffers of a prompt of T tokens, once; returns its complete pages."""
         pages = (T - self.sink_tokens) // self.block_size if T > self.sink_tokens else 0
         if self._page_min is None:
             shape = (self.geometry.num_entries, self._metadata_page_capacity(pages), self.geometry.head_dim)
             self._page_min = torch.empty(shape, dtype=self.dtype, device=self.device)
             self._page_max = torch.empty(shape, dtype=self.dtype, device=self.device)
-        if pages:
+        return pages
+
+    def _int4_rows(self, e0: int, n: int) -> Dict[str, torch.Tensor]:
+        """The INT4 buffers of entries [e0, e0 + n) that a prompt's metadata launch fills (none here)."""
+        return {}
+
+    def _build_metadata(self, entry: int, key_states: torch.Tensor) -> None:
+        """Page min/max of the prompt's complete pages (quest_offload_cache.py:276-289)."""
+        keys = key_states[0, 0]
+        if self._allocate_metadata(int(keys.shape[0])):
             kernels.build_page_metadata(keys.contiguous(), sink=self.sink_tokens, block_size=self.block_size,
                                         page_min=self._page_min[entry], page_max=self._page_max[entry])
+
+    def prompt_layer_fits(self, key_states: torch.Tensor, value_states: torch.Tensor, cos: torch.Tensor,
+                          sin: torch.Tensor) -> bool:
+        """Whether update_prompt_layer takes this layer: 16-bit K/V of the cache's type on its device, 128 channels,
+        16-row pages, tables that rotate them -- and per-entry methods that no subclass or instance replaces."""
+        own = type(self).__module__.startswith(__package__ + ".")
+        return (own and not _PROMPT_HOOKS & vars(self).keys() and key_states.shape[2] > 1
+                and key_states.dtype == self.dtype and key_states.device == self.device and self.block_size == 16
+                and key_states.shape[3] == self.geometry.head_dim == 128
+                and kernels.prefill_attention_fits(key_states, key_states, value_states, 1.0)
+                and kernels.rope_tables_fit(key_states, cos, sin))
+
+    def update_prompt_layer(self, entry0: int, key_states: torch.Tensor, value_states: torch.Tensor,
+                            cos: torch.Tensor, sin: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
+        """The prefill `update` of entries [entry0, entry0 + G) in one launch, for K/V [1, G, S, D] with K before its
+        rotary embedding (prompt_layer_fits): rotation, slab write and metadata.  Returns the rotated K and V."""
+        _, G, S, D = key_states.shape
+        for e in range(entry0, entry0 + G):
+            self._advance_prompt(e, S)
+        pages = self._allocate_metadata(S)
+        host = self.kv_residency != "hbm"
+        if host:
+            K, V = torch.empty((2, G, S, D), dtype=self.dtype, device=self.device)
+        else:
+            K, V = self._key_cache[entry0:entry0 + G, :S], self._value_cache[entry0:entry0 + G, :S]
+        assert self._page_min is not None and self._page_max is not None
+        kernels.prompt_kv(key_states, value_states, cos, sin, K, V, sink=self.sink_tokens, block_size=self.block_size,
+                          page_min=self._page_min[entry0:entry0 + G] if pages else None,
+                          page_max=self._page_max[entry0:entry0 + G] if pages else None,
+                          **self._int4_rows(entry0, G))
+        if host:
+            for g in range(G):
+                self._write_prompt(entry0 + g, K[None, g:g + 1], V[None, g:g + 1], 0, S)
+        return K[None], V[None]
+
+    def _advance_prompt(self, entry: int, length: int) -> Tuple[int, int]:
+        """The bookkeeping of one entry's prompt (the refusals of quest_offload_cache.py:513-537)."""
+        old_length, new_length = self._advance_entry(entry, length)
+        if old_length != 0:
+            raise ValueError("chunked/multiple prefill updates are unsupported")
+        if self._prompt_length is None:
+            self._prompt_length = length
+        elif self._prompt_length != length:
+            raise RuntimeError("cache entries received unequal prompt lengths")
+        return old_length, new_length
+
+    def _advance_entry(self, entry: int, length: int) -> Tuple[int, int]:
+        lengths = self._bookkeeping.advance(entry, length)
+        self._seen_tokens = self._bookkeeping.seen_tokens
+        self._initialized[entry] = True
+        return lengths
 
     def _metadata_page_capacity(self, prompt_pages: int) -> int:
         if not self.update_metadata_on_decode:
@@ -522,21 +584,13 @@ class QuestTopKOffloadedCache(_CacheBase):
         if key_states.shape[-1] != self.geometry.head_dim or key_states.dtype != self.dtype:
             raise ValueError("K/V head_dim or dtype does not match the cache")
         append_length = int(key_states.shape[-2])
-        old_length, new_length = self._bookkeeping.advance(layer_idx, append_length)
-        self._seen_tokens = self._bookkeeping.seen_tokens
-        self._initialized[layer_idx] = True
-
         if append_length > 1:
-            if old_length != 0:
-                raise ValueError("chunked/multiple prefill updates are unsupported")
-            if self._prompt_length is None:
-                self._prompt_length = append_length
-            elif self._prompt_length != append_length:
-                raise RuntimeError("cache entries received unequal prompt lengths")
+            old_length, new_length = self._advance_prompt(layer_idx, append_length)
             self._build_metadata(layer_idx, key_states)
             self._write_prompt(layer_idx, key_states, value_states, old_length, new_length)
             return key_states, value_states
 
+        old_length, _ = self._advance_entry(layer_idx, append_length)
         query = None if cache_kwargs is None else cache_kwargs.get("query_states")
         R, D = self.num_query_heads_per_kv, self.geometry.head_dim
         if query is None or tuple(query.shape) != (1, R, 1, D):

@@ -416,27 +416,30 @@ class TwilightMatchedBudgetOffloadedCache(QuestTopKOffloadedCache):
         self._dma = None  # HostGatherPipeline of post_selection_pipeline (host slabs)
 
     # ------------------------------------------------------------ metadata
+    def _allocate_metadata(self, T: int) -> int:
+        E, D = self.geometry.num_entries, self.geometry.head_dim
+        first = self._page_min is None
+        pages = super()._allocate_metadata(T)
+        if first:
+            rows = max(T, self.geometry.max_cache_len) if self.update_metadata_on_decode else T
+            self._packed = torch.empty((E, rows, D // 2), dtype=torch.uint8, device=self.device)
+            self._qscale = torch.empty((E, rows), dtype=self.dtype, device=self.device)
+            self._qmin = torch.empty_like(self._qscale)
+        return pages
+
+    def _int4_rows(self, e0: int, n: int) -> Dict[str, torch.Tensor]:
+        assert self._packed is not None and self._qscale is not None and self._qmin is not None
+        return dict(packed=self._packed[e0:e0 + n], scale=self._qscale[e0:e0 + n], minimum=self._qmin[e0:e0 + n])
+
     def _build_metadata(self, entry: int, key_states: torch.Tensor) -> None:
         """Page min/max and per-token INT4 keys of the prompt in one launch
         (twilight_offload_cache.py:925-936)."""
         keys = key_states[0, 0].contiguous()
-        T = int(keys.shape[0])
-        E, D = self.geometry.num_entries, self.geometry.head_dim
-        pages = (T - self.sink_tokens) // self.block_size if T > self.sink_tokens else 0
-        if self._page_min is None:
-            rows = max(T, self.geometry.max_cache_len) if self.update_metadata_on_decode else T
-            self._page_min = torch.empty((E, self._metadata_page_capacity(pages), D), dtype=self.dtype,
-                                         device=self.device)
-            self._page_max = torch.empty_like(self._page_min)
-            self._packed = torch.empty((E, rows, D // 2), dtype=torch.uint8, device=self.device)
-            self._qscale = torch.empty((E, rows), dtype=self.dtype, device=self.device)
-            self._qmin = torch.empty_like(self._qscale)
-        assert self._packed is not None and self._qscale is not None and self._qmin is not None
+        pages = self._allocate_metadata(int(keys.shape[0]))
         kernels.build_page_metadata(keys, sink=self.sink_tokens, block_size=self.block_size,
                                     page_min=self._page_min[entry] if pages else None,
                                     page_max=self._page_max[entry] if pages else None,
-                                    packed=self._packed[entry], scale=self._qscale[entry],
-                                    minimum=self._qmin[entry])
+                                    **{k: t[0] for k, t in self._int4_rows(entry, 1).items()})
 
     def _update_decode_metadata(self, entries: Sequence[int], position: int) -> None:
         """The decode row's INT4 code and the page it completes, if any."""
