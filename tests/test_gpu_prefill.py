@@ -40,8 +40,10 @@ def _reference(q, k, v, scale):
 @pytest.mark.parametrize("S,G,R", [(1, 1, 1), (2, 8, 4), (31, 2, 3), (32, 1, 2), (33, 2, 2), (63, 1, 1), (64, 2, 2),
                                    (65, 1, 8), (127, 4, 7), (128, 1, 1), (129, 2, 2), (255, 1, 2), (513, 2, 4),
                                    (1500, 1, 2),
-                                   # 8 wavefronts a block from 2048 blocks of 256 rows
-                                   (1, 128, 16), (256, 256, 8), (257, 128, 8)])
+                                   # the wide kernel, from 512 blocks of 256 rows on: one key tile to several, every
+                                   # parity of the last one, wavefronts that end before others
+                                   (1, 128, 16), (256, 256, 8), (257, 128, 8), (31, 64, 8), (64, 128, 4), (65, 64, 8),
+                                   (127, 64, 8), (129, 128, 4), (193, 64, 8), (320, 64, 8), (449, 64, 8), (577, 32, 8)])
 def test_prefill_attention(S, G, R, dtype):
     from headinfer import kernels
 
@@ -70,6 +72,28 @@ def test_prefill_attention_rising_scores_and_infinities():
     assert torch.equal(out.isnan().any(dim=-1), ref.isnan().any(dim=-1))
     fine = ~ref.isnan()
     assert float((out.double() - ref)[fine].abs().max()) <= 3 * U[torch.bfloat16] * float(v.double().abs().max())
+
+
+def test_wide_kernel_rising_scores_and_infinities():
+    """The same of the wide kernel: the maximum moves on every tile, and an infinite key row among later finite ones."""
+    from headinfer import kernels
+
+    S, G, R = 600, 64, 4  # 768 blocks of 256 rows
+    q, k, v = _inputs(S, 1, 1, torch.bfloat16, seed=6)
+    ramp = torch.linspace(0.0, 4.0, S, device="cuda").to(torch.bfloat16)
+    k = k + q[:, :, -1:] * ramp[None, None, :, None]
+    q = q * 0 + q[:, :, -1:]
+    for inf in (False, True):
+        if inf:
+            k[:, :, 250] = math.inf
+        ref = _reference(q, k, v, 128 ** -0.5)
+        out = kernels.prefill_attention(*(t.expand(-1, h, -1, -1).contiguous() for t, h in ((q, G * R), (k, G), (v, G))),
+                                        128 ** -0.5).view(1, S, G * R, 128)
+        assert torch.equal(out, out[:, :, :1].expand_as(out)) or inf
+        out = out[:, :, 0]
+        assert torch.equal(out.isnan().any(dim=-1), ref.isnan().any(dim=-1))
+        fine = ~ref.isnan()
+        assert float((out.double() - ref)[fine].abs().max()) <= 3 * U[torch.bfloat16] * float(v.double().abs().max())
 
 
 def test_prefill_dispatch_matches_the_general_path():

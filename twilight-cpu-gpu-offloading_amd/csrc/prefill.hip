@@ -2,11 +2,10 @@
 // fp16 / bf16): every query row attends to the key rows at or before it, the
 // attention the reference's prefill runs (mp.py:475-482).
 //
-// One block owns NW wavefronts x 32 query rows of one query head and walks the
-// key rows in tiles of 64, the next tile's loads in flight (registers, then
-// the other LDS buffer) while the current one is computed.  The products are
-// taken transposed, so that a query stays in one lane column from the scores
-// to the output:
+// A wavefront owns 32 query rows of one query head; its block walks the key rows
+// in tiles of 64, the next tile's loads in flight (registers, then the other LDS
+// buffer) while the current one is computed.  The products are taken transposed,
+// so that a query stays in one lane column from the scores to the output:
 //
 //   S^T = K Q^T    v_mfma_f32_32x32x16: A = 32 key rows, B = 32 query rows
 //   O^T += V^T P^T the same shape: A = 32 channels, B = the 32 query columns
@@ -19,15 +18,19 @@
 // the contraction takes that key order on both sides, the V^T fragment being
 // two transposing LDS reads of 4 keys each.
 //
-// Bound: the matrix cores and, beside them, the exponentials (32 a lane and
-// tile, as many issue cycles as half the tile's MFMAs).  8 KV heads of 4 query
-// heads, bf16, 32768 rows: 9.0 ms, 975 TFLOP/s of the causal half (a library
-// product of 8192^3 reaches 1186 here), against 137 ms for the score tiles in
-// fp32 through batched products, mask and softmax; 2048 rows: 60 us against
-// 1.0 ms.  Two 32-row query tiles a wavefront (half the LDS reads a product,
-// one wavefront a SIMD) took 10.5 ms and 91 us: the second wavefront of a
-// SIMD, whose products run under the first one's exponentials, is worth more.
+// Bound: the matrix cores and, beside them, the vector unit (a score costs a
+// multiply-add, an exponential, a sum, half a conversion and half a maximum: as
+// many issue cycles as its share of the products).  8 KV heads of 4 query heads,
+// bf16: 32768 rows 8.3 ms, 1060 TFLOP/s of the causal half (a library product of
+// 8192^3 reaches 1186 here), against 137 ms for the score tiles in fp32 through
+// batched products, mask and softmax; 2048 rows 69 us against 1.0 ms.  The
+// matrix cores are busy 53% of that time, at 1.9 GHz under this load.  Two 32-row
+// query tiles a wavefront (half the LDS reads a product, one wavefront a SIMD)
+// took 10.5 ms; wavefronts 4 .. 7 a product phase behind 0 .. 3, with a barrier
+// a phase, 8.7 ms.
 #pragma clang fp contract(off)
+
+#include <type_traits>
 
 #include "rope.h"
 #include "tw_common.h"
@@ -80,12 +83,19 @@ struct Frag<BF16> {
   static __device__ __forceinline__ auto narrow(float x) { return static_cast<__bf16>(x); }
 };
 
-// LDS slot (in 16-byte units) of unit u of tile row r: a row is 256 bytes, one
-// turn of the 64 banks, so unit u of 8 consecutive rows goes to 8 different
-// slots (the fragment reads of K: 8 rows, one unit), and the unit pairs of 4
-// consecutive rows to 4 different slot pairs (the transposing reads of V).
-__device__ __forceinline__ int slot(int r, int u) { return r * kRowUnits + (u ^ (2 * (r & 7))); }
+// LDS slot (in 16-byte units) of unit u of tile row r.  A row is 256 bytes, one
+// turn of the 64 banks: the units of 16 consecutive rows go to 16 different
+// slots (a fragment read of K: 16 rows, one unit), and the four units of 4
+// consecutive rows to different slot quadruples (the transposing reads of V).
+__device__ __forceinline__ int slot(int r, int u) {
+  return r * kRowUnits + (u ^ (((r & 3) << 2) | ((r >> 2) & 3)));
+}
 
+// (v_max3_f32; fmaxf would first quiet every operand, an instruction each)
+__device__ __forceinline__ float max3(float a, float b, float c) {
+  const float inf = __builtin_inff();
+  return __builtin_amdgcn_fmed3f(__builtin_amdgcn_fmed3f(a, b, inf), c, inf);
+}
 __device__ __forceinline__ float both_halves_max(float x) {
   const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
   return fmaxf(__uint_as_float(h[0]), __uint_as_float(h[1]));
@@ -95,30 +105,12 @@ __device__ __forceinline__ float both_halves_sum(float x) {
   return __uint_as_float(h[0]) + __uint_as_float(h[1]);
 }
 
-template <typename DT, int NW>
-__global__ __launch_bounds__(NW * kWave, 2) void prefill_attn_kernel(PrefillArgs a) {
+// Q^T fragments of query row `row`, rotated if the tables are given.
+template <typename DT>
+__device__ __forceinline__ void load_queries(const PrefillArgs& a, int head, int row, int half,
+                                             typename Frag<DT>::type (&qf)[8]) {
   typedef typename Frag<DT>::type frag;
-  constexpr int kLoads = kKeys * kRowUnits / (NW * kWave);  // 16-byte units a thread stages, for K and for V
-  __shared__ u32x4 s_k[2][kKeys * kRowUnits];
-  __shared__ u32x4 s_v[2][kKeys * kRowUnits];
-
-  const int tid = threadIdx.x, lane = tid % kWave, wave = wave_uniform(tid / kWave);
-  const int col = lane % 32, half = lane / 32;
-  // group-minor, the longest query tiles first
-  const int g = blockIdx.x % a.G;
-  const int rest = blockIdx.x / a.G;
-  const int head = g * a.R + rest % a.R;
-  const int qt = a.tiles - 1 - rest / a.R;
-  const int q_block = qt * NW * kQ;
-  const int q0 = q_block + wave * kQ;
   const int S = a.S;
-
-  const uint16_t* kg = a.k + g * a.k_head;
-  const uint16_t* vg = a.v + g * a.v_head;
-
-  // Q^T fragments, kept in registers
-  frag qf[8];
-  const int row = q0 + col;
   const uint16_t* qp = a.q + head * a.q_head + static_cast<int64_t>(row < S ? row : S - 1) * a.q_row + 8 * half;
 #pragma unroll
   for (int s = 0; s < 8; ++s) qf[s] = __builtin_bit_cast(frag, *reinterpret_cast<const u32x4*>(qp + 16 * s));
@@ -144,6 +136,35 @@ __global__ __launch_bounds__(NW * kWave, 2) void prefill_attn_kernel(PrefillArgs
       qf[s + 4] = __builtin_bit_cast(frag, ry);
     }
   }
+}
+
+// A block of 4 wavefronts, each taking a tile's scores, weights and values in
+// turn; two blocks share a CU and drift apart.
+template <typename DT>
+__global__ __launch_bounds__(4 * kWave, 2) void prefill_attn_kernel(PrefillArgs a) {
+  typedef typename Frag<DT>::type frag;
+  constexpr int NW = 4;
+  constexpr int kLoads = kKeys * kRowUnits / (NW * kWave);  // 16-byte units a thread stages, for K and for V
+  __shared__ u32x4 s_k[2][kKeys * kRowUnits];
+  __shared__ u32x4 s_v[2][kKeys * kRowUnits];
+
+  const int tid = threadIdx.x, lane = tid % kWave, wave = wave_uniform(tid / kWave);
+  const int col = lane % 32, half = lane / 32;
+  // group-minor, the longest query tiles first
+  const int g = blockIdx.x % a.G;
+  const int rest = blockIdx.x / a.G;
+  const int head = g * a.R + rest % a.R;
+  const int qt = a.tiles - 1 - rest / a.R;
+  const int q_block = qt * NW * kQ;
+  const int q0 = q_block + wave * kQ;
+  const int S = a.S;
+
+  const uint16_t* kg = a.k + g * a.k_head;
+  const uint16_t* vg = a.v + g * a.v_head;
+
+  const int row = q0 + col;
+  frag qf[8];
+  load_queries<DT>(a, head, row, half, qf);
 
   const int last_row = q_block + NW * kQ - 1;
   const int n_keys = (last_row < S ? last_row : S - 1) + 1;
@@ -203,9 +224,13 @@ __global__ __launch_bounds__(NW * kWave, 2) void prefill_attn_kernel(PrefillArgs
           for (int i = 0; i < 16; ++i)
             if (32 * kb + (i % 4) + 8 * (i / 4) > limit) sc[kb][i] = -__builtin_inff();
       }
-      float mx = fmaxf(sc[0][0], sc[1][0]);
+      float mx = max3(sc[0][0], sc[1][0], sc[0][1]), mx1 = max3(sc[1][1], sc[0][2], sc[1][2]);
 #pragma unroll
-      for (int i = 1; i < 16; ++i) mx = fmaxf(mx, fmaxf(sc[0][i], sc[1][i]));
+      for (int i = 3; i < 15; i += 2) {
+        mx = max3(mx, sc[0][i], sc[1][i]);
+        mx1 = max3(mx1, sc[0][i + 1], sc[1][i + 1]);
+      }
+      mx = fmaxf(max3(mx, sc[0][15], sc[1][15]), mx1);
       mx = both_halves_max(mx);
       if (__any(mx > m + slack)) {
         const float mn = fmaxf(m, mx);
@@ -276,21 +301,293 @@ __global__ __launch_bounds__(NW * kWave, 2) void prefill_attn_kernel(PrefillArgs
   }
 }
 
-template <typename DT, int NW>
-int launch(PrefillArgs a, hipStream_t s) {
-  a.tiles = (a.S + NW * kQ - 1) / (NW * kQ);
-  hipLaunchKernelGGL((prefill_attn_kernel<DT, NW>), dim3(a.tiles * a.G * a.R), dim3(NW * kWave), 0, s, a);
-  return tw_host::check_launch();
+// Blocks of 8 wavefronts, with the three streams of neighbouring tiles
+// interleaved in each wavefront.  Against the kernel above at the same block
+// size (32768 rows of 32 heads): 17.2 M cycles and 8.9 ms, 15.8 M and 8.3 ms.
+constexpr int kWideWaves = 8;
+constexpr int kWideThreads = kWideWaves * kWave;
+constexpr int kWideRows = kWideWaves * kQ;                      // query rows of a block
+template <typename DT>
+__global__ __launch_bounds__(kWideThreads, 2) void prefill_attn_wide(PrefillArgs a) {
+  typedef typename Frag<DT>::type frag;
+  __shared__ u32x4 s_tiles[4 * kKeys * kRowUnits];  // K tiles of even and odd index, then V's
+
+  const int tid = threadIdx.x, lane = tid % kWave, wave = wave_uniform(tid / kWave);
+  const int col = lane % 32, half = lane / 32;
+  // group-minor, the longest query tiles first
+  const int g = blockIdx.x % a.G;
+  const int rest = blockIdx.x / a.G;
+  const int head = g * a.R + rest % a.R;
+  const int qt = a.tiles - 1 - rest / a.R;
+  const int q_block = qt * kWideRows;
+  const int q0 = q_block + wave * kQ;
+  const int S = a.S;
+
+  const uint16_t* kg = a.k + g * a.k_head;
+  const uint16_t* vg = a.v + g * a.v_head;
+
+  const int row = q0 + col;
+  frag qf[8];
+  load_queries<DT>(a, head, row, half, qf);
+
+  const int last_row = q_block + kWideRows - 1;
+  const int n_keys = (last_row < S ? last_row : S - 1) + 1;
+  const int n_tiles = (n_keys + kKeys - 1) / kKeys;
+
+  // tiles that some row of the wavefront sees
+  const int w_tiles = (q0 + kQ - 1) / kKeys + 1 < n_tiles ? (q0 + kQ - 1) / kKeys + 1 : n_tiles;
+
+  // staging: the tile's base is wave-uniform, a thread's rows are 32-bit byte offsets from it
+  const int st_row = tid / kRowUnits, st_unit = tid % kRowUnits;
+  const int all_tiles = (S + kKeys - 1) / kKeys;
+  constexpr int kLoads = kKeys * kRowUnits / kWideThreads;  // 16-byte units a thread stages, for K and for V
+  u32x4 rk[kLoads], rv[kLoads];
+  auto load_rows = [&](const uint16_t* base, int64_t stride, int t, u32x4 (&x)[kLoads]) {
+    // past the prompt: real rows, whose keys are masked or whose tile is not read
+    const int tile = t < all_tiles ? t : all_tiles - 1;
+    const char* p = reinterpret_cast<const char*>(base + static_cast<int64_t>(tile) * kKeys * stride);
+    const int last = S - 1 - tile * kKeys;
+    const uint32_t bytes = static_cast<uint32_t>(stride) * 2, end = (last < kKeys ? last : kKeys) * bytes;
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) {
+      uint32_t at = static_cast<uint32_t>(st_row + i * (kKeys / kLoads)) * bytes;
+      at = at < end ? at : end;
+      x[i] = *reinterpret_cast<const u32x4*>(p + (at + 16u * st_unit));
+    }
+  };
+  const int st_at = slot(st_row, st_unit);  // rows kKeys / kLoads apart share the swizzle
+  static_assert((kKeys / kLoads) % 16 == 0, "the swizzle repeats every 16 rows");
+  auto store_rows = [&](int tile, const u32x4 (&x)[kLoads]) {
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) s_tiles[st_at + (tile * kKeys + i * (kKeys / kLoads)) * kRowUnits] = x[i];
+  };
+
+  f32x16 o[4], sc[2];
+  frag p_even[4], p_odd[4];
+  f32x16 zero = {0.0f};
+  asm volatile("" : "+v"(zero));  // kept in registers: the first product of every chain adds to it
+  float m = -__builtin_inff(), l = 0.0f;
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) o[c][i] = 0.0f;
+  // raw scores past the running maximum by less than this are taken without
+  // moving it: their weights stay below 2^8, and the accumulators are not
+  // rescaled on every tile
+  const float slack = 8.0f / a.scale_log2;
+
+  // fragment addresses in the first tile; the tile and the rest of the row index are immediates
+  typedef __attribute__((address_space(3))) char* lds_ptr;
+  const lds_ptr lds = (lds_ptr)(reinterpret_cast<uintptr_t>(s_tiles));
+  lds_ptr k_at[8], v_at[4][2];
+#pragma unroll
+  for (int s = 0; s < 8; ++s) k_at[s] = lds + 16 * slot(col, 2 * s + half);
+  // V^T fragments: lane i of a 16-lane group names key row i / 4 and channels 4 (i % 4) .. + 3
+  const int vrow = 4 * half + (lane % 16) / 4;
+  const int vch = 16 * ((lane / 16) % 2) + 4 * (lane % 4);
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) v_at[c][h] = lds + 16 * slot(8 * h + vrow, (32 * c + vch) / 8) + 8 * ((vch % 8) / 4);
+  constexpr int kTileBytes = kKeys * 256;
+  auto key_frag = [&](int tile, int j) {  // K fragment j of 16: 32 keys x 16 channels
+    return *(__attribute__((address_space(3))) frag*)(k_at[j % 8] + tile * kTileBytes + (j / 8) * 32 * 256);
+  };
+  auto value_frag = [&](int tile, int j) {  // V^T fragment j of 16: 16 keys x 32 channels
+    s16x8 x;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const s16x4 y = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(
+          v_at[j % 4][h] + tile * kTileBytes + (j / 4) * 16 * 256));
+#pragma unroll
+      for (int i = 0; i < 4; ++i) x[4 * h + i] = y[i];
+    }
+    return __builtin_bit_cast(frag, x);
+  };
+  auto stage = [&](int t, int parity) {  // iteration t's share of the tiles to come
+    store_rows(parity, rk);
+    store_rows(2 + parity, rv);
+    load_rows(kg, a.k_row, t + 3, rk);
+    load_rows(vg, a.v_row, t + 1, rv);
+  };
+
+  // Iteration t takes the weights of tile t on the vector unit while the
+  // matrix cores form the scores of tile t + 1 and then the values of tile
+  // t - 1.  The three streams are independent and interleaved by hand, a
+  // matrix instruction and a few vector instructions a step (a wavefront's
+  // products and exponentials one after the other leave either unit idle half
+  // the time, with two wavefronts on the SIMD too).  It stores K tile t + 2 and
+  // V tile t over K t and V t - 2, which iteration t - 1 read last.  LAST: the
+  // tile holds keys in the future of some row -- the last of the wavefront's
+  // tiles, and no other.
+  auto iteration = [&](int t, auto parity, auto first, auto last, const frag (&pf)[4], frag (&pn)[4]) __attribute__((always_inline)) {
+    constexpr int PAR = decltype(parity)::value;  // of t
+    constexpr bool FIRST = decltype(first)::value, LAST = decltype(last)::value;
+    constexpr int kAhead = 3;  // steps between a fragment's LDS read and its use
+    constexpr int kMaxSteps = 4;
+    // first weight of step j: scores 0 .. 15 before step 16, from which their registers take the next tile's, the
+    // others before step 24
+    auto exp_begin = [](int j) { return j <= 16 ? (j - kMaxSteps - 1) * 16 / (15 - kMaxSteps) : j < 24 ? 2 * j - 16 : 32; };
+    frag ring[kAhead + 1];
+    auto fetch = [&](int j) {
+      if (j < 16) {
+        if constexpr (!FIRST) ring[j % (kAhead + 1)] = value_frag(2 + (PAR ^ 1), j);
+      } else if (j < 32) {
+        if constexpr (!LAST) ring[j % (kAhead + 1)] = key_frag(PAR ^ 1, j - 16);
+      }
+    };
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) fetch(j);
+    if constexpr (LAST) {
+      const int limit = row - t * kKeys - 4 * half;
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+          if (32 * kb + (i % 4) + 8 * (i / 4) > limit) sc[kb][i] = -__builtin_inff();
+    }
+    float mx = -__builtin_inff(), f = 1.0f, ms = 0.0f, sum = 0.0f, p0 = 0.0f;
+    bool moved = false;
+    uint32_t pw[16];
+#pragma unroll
+    for (int j = 0; j < 32; ++j) {
+      __builtin_amdgcn_sched_barrier(0);
+      fetch(j + kAhead);
+      if (j < 16) {
+        if constexpr (!FIRST) o[j % 4] = Frag<DT>::mfma(ring[j % (kAhead + 1)], pf[j / 4], o[j % 4]);
+      } else {
+        if constexpr (!LAST)
+          sc[j / 8 - 2] = Frag<DT>::mfma(ring[j % (kAhead + 1)], qf[j % 8], j % 8 == 0 ? zero : sc[j / 8 - 2]);
+      }
+      if (j < kMaxSteps) {
+#pragma unroll
+        for (int i = 4 * j; i < 4 * j + 4; ++i) mx = max3(mx, sc[0][i], sc[1][i]);
+      } else if (j == kMaxSteps) {
+        mx = both_halves_max(mx);
+        moved = __any(mx > m + slack);
+        const float mn = moved ? fmaxf(m, mx) : m;
+        // an unmoved maximum keeps its sums (-inf - -inf is not a factor)
+        f = m == mn ? 1.0f : __builtin_amdgcn_exp2f((m - mn) * a.scale_log2);
+        m = mn;
+        ms = m * a.scale_log2;
+      } else {
+#pragma unroll
+        for (int i = exp_begin(j); i < exp_begin(j + 1); ++i) {
+          const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[i / 16][i % 16], a.scale_log2, -ms));
+          sum += p;
+          if (i % 2 == 0)
+            p0 = p;
+          else
+            pw[i / 2] = narrow_pair(p0, p, DT{});
+          // (formed here, not where they are used after the branch below)
+          if (i % 2 == 1) asm volatile("" : "+v"(pw[i / 2]), "+v"(sum));
+        }
+      }
+      if (j == 1) stage(t, PAR);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    l = l * f + sum;
+    if (moved) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[c][i] *= f;
+    }
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      const u32x4 w = {pw[4 * ks], pw[4 * ks + 1], pw[4 * ks + 2], pw[4 * ks + 3]};
+      pn[ks] = __builtin_bit_cast(frag, w);
+    }
+  };
+
+  load_rows(kg, a.k_row, 0, rk);
+  store_rows(0, rk);
+  load_rows(kg, a.k_row, 1, rk);
+  store_rows(1, rk);
+  load_rows(kg, a.k_row, 2, rk);
+  load_rows(vg, a.v_row, 0, rv);
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < 16; ++j)
+    sc[j / 8] = Frag<DT>::mfma(key_frag(0, j), qf[j % 8], j % 8 == 0 ? zero : sc[j / 8]);
+  __syncthreads();  // iteration 0 stores over K tile 0
+  constexpr std::integral_constant<int, 0> even{};
+  constexpr std::integral_constant<int, 1> odd{};
+  constexpr std::true_type yes{};
+  constexpr std::false_type no{};
+  // an even iteration reads p_odd and leaves p_even
+  if (w_tiles == 1)
+    iteration(0, even, yes, yes, p_odd, p_even);
+  else
+    iteration(0, even, yes, no, p_odd, p_even);
+  __syncthreads();
+  int t = 1;
+  for (; t + 1 < w_tiles - 1; t += 2) {
+    iteration(t, odd, no, no, p_even, p_odd);
+    __syncthreads();
+    iteration(t + 1, even, no, no, p_odd, p_even);
+    __syncthreads();
+  }
+  if (t < w_tiles - 1) {
+    iteration(t, odd, no, no, p_even, p_odd);
+    __syncthreads();
+    ++t;
+  }
+  auto finish = [&](int tile, const frag (&pf)[4]) {
+#pragma unroll
+    for (int j = 0; j < 16; ++j) o[j % 4] = Frag<DT>::mfma(value_frag(tile, j), pf[j / 4], o[j % 4]);
+  };
+  if (w_tiles % 2 != 0) {  // the last tile's index is even
+    if (w_tiles > 1) {
+      iteration(t, even, no, yes, p_odd, p_even);
+      __syncthreads();
+    }
+    finish(2, p_even);
+  } else {
+    iteration(t, odd, no, yes, p_even, p_odd);
+    __syncthreads();
+    finish(3, p_odd);
+  }
+  for (t = w_tiles; t < n_tiles; ++t) {  // the block's later wavefronts go on
+    stage(t, t & 1);
+    __syncthreads();
+  }
+
+  const float inv = 1.0f / both_halves_sum(l);
+  if (row < S) {
+    uint16_t* p = a.out + static_cast<int64_t>(row) * a.out_row + head * kHead + 4 * half;
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        typename Frag<DT>::quad w;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) w[j] = Frag<DT>::narrow(o[c][4 * i + j] * inv);
+        *reinterpret_cast<typename Frag<DT>::quad*>(p + 32 * c + 8 * i) = w;
+      }
+  }
 }
 
-// 8 wavefronts share each staged tile where there are enough blocks to keep
-// every CU in work to the end (8 a CU); with fewer, smaller blocks balance
-// better.  32 heads: 32768 rows (4096 blocks) 9.0 ms against 9.4 with 4
-// wavefronts, 8192 rows (1024 blocks) 0.63 ms both, 2048 rows 69 us against 60.
+constexpr int kWideBlocks = 512;
+
+// The wide kernel from two blocks a CU on; with fewer, blocks of half the rows
+// balance better, and two of them on a CU overlap by themselves.  One attention
+// layer, small against wide blocks: 2048 rows of 32 heads (256 wide blocks) 245
+// against 251 us, 4096 (512) 450 and 434, 12000 of 12 (564) 726 and 684, 8192 of
+// 32 (1024) 1145 and 1075, 32768 11.0 ms (8 wavefronts) and 10.1.
 template <typename DT>
-int launch_any(const PrefillArgs& a, hipStream_t s) {
-  const int64_t wide = static_cast<int64_t>((a.S + 8 * kQ - 1) / (8 * kQ)) * a.G * a.R;
-  return wide >= 2048 ? launch<DT, 8>(a, s) : launch<DT, 4>(a, s);
+int launch(PrefillArgs a, hipStream_t s) {
+  const int heads = a.G * a.R;
+  const int wide = (a.S + kWideRows - 1) / kWideRows;
+  const int64_t far = 1 << 24;  // the wide kernel's offsets inside a tile are 32-bit
+  if (static_cast<int64_t>(wide) * heads >= kWideBlocks && a.k_row <= far && a.v_row <= far) {
+    a.tiles = wide;
+    hipLaunchKernelGGL(prefill_attn_wide<DT>, dim3(wide * heads), dim3(kWideThreads), 0, s, a);
+  } else {
+    a.tiles = (a.S + 4 * kQ - 1) / (4 * kQ);
+    hipLaunchKernelGGL(prefill_attn_kernel<DT>, dim3(a.tiles * heads), dim3(4 * kWave), 0, s, a);
+  }
+  return tw_host::check_launch();
 }
 
 }  // namespace
@@ -326,5 +623,5 @@ extern "C" int tw_prefill_attention(const void* q, const void* k, const void* v,
   a.S = S, a.G = G, a.R = R;
   a.scale_log2 = softmax_scale * 1.4426950408889634f;
   const hipStream_t s = static_cast<hipStream_t>(stream);
-  return dtype == TW_DTYPE_F16 ? launch_any<F16>(a, s) : launch_any<BF16>(a, s);
+  return dtype == TW_DTYPE_F16 ? launch<F16>(a, s) : launch<BF16>(a, s);
 }
