@@ -8,10 +8,12 @@
 // Two kernels per layer:
 //
 // 1. Scores.  A block of 8 wavefronts scores a tile of 64 pages of one KV
-//    group for all R query heads.  The tile is staged once in LDS with
-//    16-byte loads (padded, 16-byte aligned row pitch); wavefronts w and
-//    w+4 then score head w (w+4, ...) with lane = page, each summing half of
-//    the 32 accumulators, so the q > 0 choice of min or max is wave-uniform.
+//    group for all R query heads, staged in LDS with 16-byte loads (padded,
+//    16-byte aligned row pitch), lane = page.  At D = 128 a wavefront owns 4
+//    of the 32 accumulators for every head (score_order.h); otherwise
+//    wavefronts w and w + 4 score head w (w + 4, ...), each summing half of
+//    the accumulators.  Either way the q > 0 choice of min or max is
+//    wave-uniform.
 //    Order (bit-exact with the reference for D = 128): 32 accumulators,
 //    accumulator l adds the products of channels
 //    l, l+32, l+64, l+96 in that order starting from +0; the 32 accumulators
@@ -60,8 +62,9 @@ namespace {
 using namespace sel;
 
 constexpr int kTilePages = 64;
-constexpr int kScoreBlock = 512;  // score kernel: 8 wavefronts, two per head
+constexpr int kScoreBlock = 512;  // score kernels: 8 wavefronts
 constexpr int kMaxD = 256;
+constexpr unsigned int kChipCUs = 256;
 
 // ------------------------------------------------------------------ scores
 __device__ __forceinline__ float lds_load(const uint8_t* p, F16) {
@@ -191,6 +194,147 @@ __device__ __forceinline__ void tile_key_range(const ScoreArgs& a, int64_t row, 
   if (lane_id() == 0) a.tile_mm[row * tiles + p0 / kTilePages] = make_uint2(kmax, kmin);
 }
 
+// The launch's bookkeeping, tile `tile` of group g: arrival counters and the
+// group's union record (bitmap words 2 tile and 2 tile + 1, mask words
+// [32 tile, 32 tile + 32); every tile of the launch, a ragged group's too).
+__device__ __forceinline__ void clear_tile_state(const ScoreArgs& a, int g, int tile) {
+  if (a.zero_counters != nullptr && g == 0 && tile == 0) {
+    for (int i = static_cast<int>(threadIdx.x); i < a.n_counters; i += kScoreBlock) a.zero_counters[i] = 0u;
+  }
+  if (a.rec != nullptr) {
+    uint32_t* rec = a.rec + g * a.rec_stride;
+    const int t = static_cast<int>(threadIdx.x);
+    const int mw = tile * (kTilePages / 2) + t - 2;
+    if (t < 2)
+      rec[2 * tile + t] = 0u;
+    else if (t < 2 + kTilePages / 2 && mw < union_mask_words(a.P))
+      rec[union_mask_offset(a.P) + mw] = 0u;
+  }
+}
+
+// Ragged groups: a tile past its group's pages has nothing to read.  Where the
+// launch has more blocks than the chip has CUs a block waits for its group's
+// length before it loads (other blocks fill the wait, and dead tiles cost no
+// bandwidth); a smaller launch loads beside it, up to the buffer's P pages.
+// 8 requests of 16K to 128K tokens, 4 KV heads of 4: a decode layer 71.6 -> 69.2 us.
+__device__ __forceinline__ bool waits_for_length(const ScoreArgs& a) {
+  return a.lengths != nullptr && gridDim.x > kChipCUs;
+}
+
+// Scores of one tile of kTilePages pages for R heads at D = 128 with 16-byte
+// aligned metadata, in two phases: channels [0, 64) of every page are stored
+// and scored while the loads of channels [64, 128) are still in flight.
+//
+// Bound: the vector unit where the launch has blocks for every CU, latency
+// below that.  With a wavefront per head, both rows were read from LDS, chosen
+// from and widened again for every head: the score launch of 8 requests of 16K
+// to 128K tokens, 4 KV heads of 7, took 52.0 us, now 34.2; one request of 32K,
+// 8 KV heads of 8, the whole layer 31.0 -> 29.9 us.  At 4 heads and fewer every
+// wavefront of the other form has a head of its own and it stays ahead: the
+// 32K Quest layer of 4 heads 23.17 against 23.22 us, the fused Twilight score of
+// 4 and of 6 heads 37.8 against 38.2 and 40.5 against 41.0 us a layer.
+template <typename DT, int R>
+__global__ __launch_bounds__(kScoreBlock) void quest_score_tile_kernel(ScoreArgs a) {
+  using S = typename DT::storage;
+  constexpr int D = 128;
+  constexpr int es = static_cast<int>(sizeof(S));
+  constexpr int kQuads = D * es / 16;  // 16-byte quads per row
+  constexpr int kHq = kQuads / 2;
+  constexpr int kPerHalf = 2 * kTilePages * kHq / kScoreBlock;
+  constexpr int pitch = D * es + 16;
+  static_assert(kPerHalf * kScoreBlock == 2 * kTilePages * kHq && kScoreBlock == kScoreWaves * kWave, "tile shape");
+  extern __shared__ __align__(16) uint8_t lds[];
+  float* part = reinterpret_cast<float*>(lds + 2 * kTilePages * pitch);  // [8][R][64]
+  // group-minor: workgroups go to the XCDs round-robin, so with G a multiple
+  // of 8 group g's blocks of every launch of the layer share XCD g % 8 (and
+  // its L2)
+  const int g = static_cast<int>(blockIdx.x) % a.G;
+  const int tile = static_cast<int>(blockIdx.x) / a.G;
+  const int p0 = tile * kTilePages;
+  const int tid = static_cast<int>(threadIdx.x);
+  const float* qg = a.q + static_cast<int64_t>(g) * R * D;
+  const S* mn = static_cast<const S*>(a.pmin) + g * a.group_stride + static_cast<int64_t>(p0) * D;
+  const S* mx = static_cast<const S*>(a.pmax) + g * a.group_stride + static_cast<int64_t>(p0) * D;
+  // (an unconditional load: without lengths it reads the first query word
+  // and ignores it)
+  const int length = *(a.lengths != nullptr ? a.lengths + g : reinterpret_cast<const int32_t*>(a.q));
+  int P = a.P;
+  if (waits_for_length(a)) {
+    P = ragged_pages(length, a.sink, a.recent, a.bs, a.P);
+    if (p0 >= P) {  // block-uniform
+      clear_tile_state(a, g, tile);
+      return;
+    }
+  }
+  // Loads are unconditional (indices clamped into the tile), so they issue
+  // back to back and each store waits only for its own load.
+  const int np_cap = (P - p0) < kTilePages ? (P - p0) : kTilePages;
+  const int total_h = 2 * np_cap * kHq;
+  uint4 va[kPerHalf], vb[kPerHalf];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+#pragma unroll
+    for (int j = 0; j < kPerHalf; ++j) {
+      int i = tid + j * kScoreBlock;
+      i = i < total_h ? i : total_h - 1;
+      const bool which = i >= np_cap * kHq;
+      const int rem = i - (which ? np_cap * kHq : 0);
+      const int page = rem / kHq;
+      const int qd = rem % kHq + h * kHq;
+      const uint4 v = load_stream(reinterpret_cast<const uint4*>(which ? mx : mn) + page * kQuads + qd);
+      if (h == 0) va[j] = v; else vb[j] = v;
+    }
+    // the first half's loads go out first (and so arrive first)
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  clear_tile_state(a, g, tile);
+  auto store_half = [&](int h, const uint4 (&v)[kPerHalf]) {
+#pragma unroll
+    for (int j = 0; j < kPerHalf; ++j) {
+      // clamped like the loads: a thread past the tile stores the last
+      // quad's value to the last quad's place again
+      int i = tid + j * kScoreBlock;
+      i = i < total_h ? i : total_h - 1;
+      const bool which = i >= np_cap * kHq;
+      const int rem = i - (which ? np_cap * kHq : 0);
+      const int page = rem / kHq;
+      const int qd = rem % kHq + h * kHq;
+      *reinterpret_cast<uint4*>(lds + ((which ? kTilePages : 0) + page) * pitch + qd * 16) = v[j];
+    }
+  };
+  store_half(0, va);
+  if (a.lengths != nullptr) {
+    P = ragged_pages(length, a.sink, a.recent, a.bs, a.P);
+    if (p0 >= P) return;  // block-uniform
+  }
+  const int np = (P - p0) < kTilePages ? (P - p0) : kTilePages;
+  __syncthreads();
+  const int wave = wave_uniform(tid / kWave);
+  const int lane = lane_id();
+  const uint8_t* min_row = lds + lane * pitch;
+  const uint8_t* max_row = lds + (kTilePages + lane) * pitch;
+  float acc[R][4];
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[r][i] = 0.0f;
+  score_chunks<DT, R, 0, 2>(min_row, max_row, wave, qg, acc);
+  store_half(1, vb);
+  __syncthreads();
+  score_chunks<DT, R, 2, 4>(min_row, max_row, wave, qg, acc);
+  score_store_parts<R>(part, wave, lane, acc);
+  __syncthreads();
+  if (wave < R) {
+    const float sc = score_combine<R>(part, wave, lane);
+    const int64_t row = static_cast<int64_t>(g) * R + wave;
+    if (lane < np) {
+      a.scores[row * a.score_stride + p0 + lane] = sc;
+      if (a.scores_out != nullptr) a.scores_out[row * a.P + p0 + lane] = sc;
+    }
+    if (a.tile_mm != nullptr) tile_key_range(a, row, p0, lane < np, sc);
+  }
+}
+
 // Scores of one tile for D = DFIX and at most 4 heads, in two phases:
 // channels [0, DFIX/2) of every page are stored and scored while the loads
 // of channels [DFIX/2, DFIX) are still in flight.  Each accumulator takes
@@ -304,33 +448,26 @@ __device__ void score_tile_split(const ScoreArgs& a, int g, int p0, int np_cap, 
   }
 }
 
-// Scores of one tile of kTilePages pages of group g for all R heads.
+// Scores of one tile of kTilePages pages of group g for all R heads: every
+// head_dim, alignment and head count.
 template <typename DT, int DFIX>
 __device__ void score_tile(const ScoreArgs& a, int g, int tile, uint8_t* lds) {
   using S = typename DT::storage;
   const int p0 = tile * kTilePages;
   if (p0 >= a.P) return;  // block-uniform
-  if (a.zero_counters != nullptr && g == 0 && tile == 0) {
-    for (int i = static_cast<int>(threadIdx.x); i < a.n_counters; i += kScoreBlock) a.zero_counters[i] = 0u;
-  }
-  if (a.rec != nullptr) {
-    // every tile of the launch (a ragged group's too): words 2 tile and
-    // 2 tile + 1 of the bitmap, mask words [32 tile, 32 tile + 32)
-    uint32_t* rec = a.rec + g * a.rec_stride;
-    const int t = static_cast<int>(threadIdx.x);
-    const int mw = (p0 >> 1) + t - 2;
-    if (t < 2)
-      rec[2 * tile + t] = 0u;
-    else if (t < 2 + kTilePages / 2 && mw < union_mask_words(a.P))
-      rec[union_mask_offset(a.P) + mw] = 0u;
-  }
+  clear_tile_state(a, g, tile);
   // A ragged group's length is read in the same round trip as the tile: the
   // tile is staged up to the buffer's P pages (in bounds), and only the
   // scores of the group's own pages are written.
   // (an unconditional load: without lengths it reads the first query word
   // and ignores it)
   const int length = *(a.lengths != nullptr ? a.lengths + g : reinterpret_cast<const int32_t*>(a.q));
-  const int np_cap = (a.P - p0) < kTilePages ? (a.P - p0) : kTilePages;
+  int p_cap = a.P;
+  if (waits_for_length(a)) {
+    p_cap = ragged_pages(length, a.sink, a.recent, a.bs, a.P);
+    if (p0 >= p_cap) return;  // block-uniform
+  }
+  const int np_cap = (p_cap - p0) < kTilePages ? (p_cap - p0) : kTilePages;
   if constexpr (DFIX > 0) {
     const uintptr_t base = reinterpret_cast<uintptr_t>(static_cast<const S*>(a.pmin) + g * a.group_stride) |
                            reinterpret_cast<uintptr_t>(static_cast<const S*>(a.pmax) + g * a.group_stride);
@@ -1003,12 +1140,25 @@ int prepare_long_rows(SelectArgs& s, int n_rows, bool vec, uint8_t* lw, hipStrea
 template <typename DT>
 int launch_score(const ScoreArgs& a, hipStream_t stream) {
   const int tiles = (a.P + kTilePages - 1) / kTilePages;
-  const size_t lds = static_cast<size_t>(2 * kTilePages) *
-                         (static_cast<size_t>(a.D) * sizeof(typename DT::storage) + 16) +
-                     static_cast<size_t>(a.R) * a.D * sizeof(float);
-  if (lds > 160 * 1024) return TW_EUNSUPPORTED;  // gfx950: 160 KB of LDS per CU
+  const size_t tile_bytes =
+      static_cast<size_t>(2 * kTilePages) * (static_cast<size_t>(a.D) * sizeof(typename DT::storage) + 16);
   const dim3 grid(tiles * a.G);
-  auto kern = a.D == 128 ? quest_score_kernel<DT, 128> : quest_score_kernel<DT, 0>;
+  // every tile row starts on 16 bytes, and the heads' accumulators fit the registers
+  const bool aligned = ((reinterpret_cast<uintptr_t>(a.pmin) | reinterpret_cast<uintptr_t>(a.pmax)) % 16) == 0 &&
+                       (a.G == 1 || (a.group_stride * sizeof(typename DT::storage)) % 16 == 0);
+  const bool tile_path = a.D == 128 && a.R > 4 && a.R <= 8 && aligned;
+  const size_t lds =
+      tile_bytes + static_cast<size_t>(a.R) * (tile_path ? kScoreWaves * kWave : a.D) * sizeof(float);
+  if (lds > 160 * 1024) return TW_EUNSUPPORTED;  // gfx950: 160 KB of LDS per CU
+  void (*kern)(ScoreArgs) = a.D == 128 ? quest_score_kernel<DT, 128> : quest_score_kernel<DT, 0>;
+  if (tile_path) {
+    switch (a.R) {
+      case 5: kern = quest_score_tile_kernel<DT, 5>; break;
+      case 6: kern = quest_score_tile_kernel<DT, 6>; break;
+      case 7: kern = quest_score_tile_kernel<DT, 7>; break;
+      default: kern = quest_score_tile_kernel<DT, 8>; break;
+    }
+  }
   if (lds > 64 * 1024)
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                               static_cast<int>(lds));

@@ -45,5 +45,79 @@ __device__ __forceinline__ void select8(const uint8_t* mn, const uint8_t* mx, co
   for (int i = 0; i < 8; ++i) x[i] = q[i] > 0.0f ? hi[i] : lo[i];
 }
 
+// ---- the tile score of D = 128, all heads of a group in one pass (quest.hip)
+//
+// A block of 8 wavefronts scores a tile of 64 pages staged in LDS, lane = page.
+// Wavefront w owns accumulators 4 w .. 4 w + 3 of the 32 (channels d with
+// d mod 32 in that range) for every head: it reads and widens each of its
+// channels' min and max once, whatever the number of heads, where a wavefront
+// per head read both rows again for each.  The queries are wave-uniform and
+// stay in scalar registers (constant address space), so the q > 0 choice is a
+// scalar mask and a head costs three vector instructions a channel (select,
+// multiply, add).  The accumulators and their adjacent-pair tree are those of
+// the 32-accumulator order: the in-lane tree covers 4, the combine the other 8.
+constexpr int kScoreWaves = 8;
+typedef const __attribute__((address_space(4))) uint32_t* ConstWords;
+
+__device__ __forceinline__ void load4(const uint8_t* p, float (&x)[4], F16) {
+  const uint2 w = *reinterpret_cast<const uint2*>(p);
+  x[0] = to_f32(F16{}, static_cast<uint16_t>(w.x & 0xffffu));
+  x[1] = to_f32(F16{}, static_cast<uint16_t>(w.x >> 16));
+  x[2] = to_f32(F16{}, static_cast<uint16_t>(w.y & 0xffffu));
+  x[3] = to_f32(F16{}, static_cast<uint16_t>(w.y >> 16));
+}
+__device__ __forceinline__ void load4(const uint8_t* p, float (&x)[4], BF16) {
+  const uint2 w = *reinterpret_cast<const uint2*>(p);
+  x[0] = to_f32(BF16{}, static_cast<uint16_t>(w.x & 0xffffu));
+  x[1] = to_f32(BF16{}, static_cast<uint16_t>(w.x >> 16));
+  x[2] = to_f32(BF16{}, static_cast<uint16_t>(w.y & 0xffffu));
+  x[3] = to_f32(BF16{}, static_cast<uint16_t>(w.y >> 16));
+}
+__device__ __forceinline__ void load4(const uint8_t* p, float (&x)[4], F32) {
+  *reinterpret_cast<float4*>(x) = *reinterpret_cast<const float4*>(p);
+}
+
+// Adds 32-channel chunks [C0, C1) of the wavefront's residues to acc for R
+// heads.  qg: the group's q, [R][128].
+template <typename DT, int R, int C0, int C1>
+__device__ __forceinline__ void score_chunks(const uint8_t* min_row, const uint8_t* max_row, int wave, const float* qg,
+                                             float (&acc)[R][4]) {
+  constexpr int es = static_cast<int>(sizeof(typename DT::storage));
+  const ConstWords q = (ConstWords)(reinterpret_cast<uintptr_t>(qg));
+#pragma unroll
+  for (int c = C0; c < C1; ++c) {
+    const int d0 = 32 * c + 4 * wave;
+    float lo[4], hi[4];
+    load4(min_row + d0 * es, lo, DT{});
+    load4(max_row + d0 * es, hi, DT{});
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int at = r * 128 + d0;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const uint32_t qb = q[at + i];
+        const bool up = static_cast<int32_t>(qb) > 0;  // q > 0 on its bits (a NaN's product is a NaN either way)
+        acc[r][i] = acc[r][i] + (up ? hi[i] : lo[i]) * __uint_as_float(qb);
+      }
+    }
+  }
+}
+
+// The wavefronts' four-accumulator trees to part[(w * NR + r) * 64 + lane].
+template <int NR>
+__device__ __forceinline__ void score_store_parts(float* part, int wave, int lane, const float (&acc)[NR][4]) {
+#pragma unroll
+  for (int r = 0; r < NR; ++r)
+    part[(wave * NR + r) * kWave + lane] = (acc[r][0] + acc[r][1]) + (acc[r][2] + acc[r][3]);
+}
+// Head r's score of page `lane` (after a barrier).
+template <int NR>
+__device__ __forceinline__ float score_combine(const float* part, int r, int lane) {
+  float p[kScoreWaves];
+#pragma unroll
+  for (int w = 0; w < kScoreWaves; ++w) p[w] = part[(w * NR + r) * kWave + lane];
+  return ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
+}
+
 }  // namespace
 }  // namespace tw
