@@ -9,10 +9,10 @@
 //
 // 1. Scores.  A block of 8 wavefronts scores a tile of 64 pages of one KV
 //    group for all R query heads, staged in LDS with 16-byte loads (padded,
-//    16-byte aligned row pitch), lane = page.  At D = 128 a wavefront owns 4
-//    of the 32 accumulators for every head (score_order.h); otherwise
-//    wavefronts w and w + 4 score head w (w + 4, ...), each summing half of
-//    the accumulators.  Either way the q > 0 choice of min or max is
+//    16-byte aligned row pitch), lane = page.  At D = 128 and up to 8 heads a
+//    wavefront owns 4 of the 32 accumulators for every head (score_order.h);
+//    otherwise wavefronts w and w + 4 score head w (w + 4, ...), each summing
+//    half of the accumulators.  Either way the q > 0 choice of min or max is
 //    wave-uniform.
 //    Order (bit-exact with the reference for D = 128): 32 accumulators,
 //    accumulator l adds the products of channels
@@ -225,14 +225,15 @@ __device__ __forceinline__ bool waits_for_length(const ScoreArgs& a) {
 // aligned metadata, in two phases: channels [0, 64) of every page are stored
 // and scored while the loads of channels [64, 128) are still in flight.
 //
-// Bound: the vector unit where the launch has blocks for every CU, latency
-// below that.  With a wavefront per head, both rows were read from LDS, chosen
-// from and widened again for every head: the score launch of 8 requests of 16K
-// to 128K tokens, 4 KV heads of 7, took 52.0 us, now 34.2; one request of 32K,
-// 8 KV heads of 8, the whole layer 31.0 -> 29.9 us.  At 4 heads and fewer every
-// wavefront of the other form has a head of its own and it stays ahead: the
-// 32K Quest layer of 4 heads 23.17 against 23.22 us, the fused Twilight score of
-// 4 and of 6 heads 37.8 against 38.2 and 40.5 against 41.0 us a layer.
+// Bound: latency where a launch has a block a CU, instruction issue (the scalar
+// choice of min or max beside the vector work) where it has more.  With a
+// wavefront a head, both rows were read from LDS, chosen from and widened again
+// for every head, and the queries waited for in LDS: the score launch of 8
+// requests of 16K to 128K tokens, 4 KV heads of 7, took 52.0 us, now 34.0; the
+// layer of one request, 8 KV heads: 32K and 4 heads each 23.2 -> 22.9 us, 4K
+// 17.7 -> 17.1, 128K 33.7 -> 31.6; 32K and 8 heads each 31.0 -> 29.3.  (Loaded
+// one by one at their uses, the scalar queries cost 0.4 us a layer at 4 heads
+// and 0.6 at 8.  Two tiles a block, one scalar choice for both: no gain.)
 template <typename DT, int R>
 __global__ __launch_bounds__(kScoreBlock) void quest_score_tile_kernel(ScoreArgs a) {
   using S = typename DT::storage;
@@ -287,6 +288,9 @@ __global__ __launch_bounds__(kScoreBlock) void quest_score_tile_kernel(ScoreArgs
     // the first half's loads go out first (and so arrive first)
     __builtin_amdgcn_sched_barrier(0);
   }
+  const int wave = wave_uniform(tid / kWave);
+  ScoreQ<R> q;
+  q.load(qg, wave, 0);
   clear_tile_state(a, g, tile);
   auto store_half = [&](int h, const uint4 (&v)[kPerHalf]) {
 #pragma unroll
@@ -309,7 +313,6 @@ __global__ __launch_bounds__(kScoreBlock) void quest_score_tile_kernel(ScoreArgs
   }
   const int np = (P - p0) < kTilePages ? (P - p0) : kTilePages;
   __syncthreads();
-  const int wave = wave_uniform(tid / kWave);
   const int lane = lane_id();
   const uint8_t* min_row = lds + lane * pitch;
   const uint8_t* max_row = lds + (kTilePages + lane) * pitch;
@@ -318,128 +321,16 @@ __global__ __launch_bounds__(kScoreBlock) void quest_score_tile_kernel(ScoreArgs
   for (int r = 0; r < R; ++r)
 #pragma unroll
     for (int i = 0; i < 4; ++i) acc[r][i] = 0.0f;
-  score_chunks<DT, R, 0, 2>(min_row, max_row, wave, qg, acc);
+  score_chunks<DT, R, 0>(min_row, max_row, wave, q, acc);
+  q.load(qg, wave, 2);
   store_half(1, vb);
   __syncthreads();
-  score_chunks<DT, R, 2, 4>(min_row, max_row, wave, qg, acc);
+  score_chunks<DT, R, 2>(min_row, max_row, wave, q, acc);
   score_store_parts<R>(part, wave, lane, acc);
   __syncthreads();
   if (wave < R) {
     const float sc = score_combine<R>(part, wave, lane);
     const int64_t row = static_cast<int64_t>(g) * R + wave;
-    if (lane < np) {
-      a.scores[row * a.score_stride + p0 + lane] = sc;
-      if (a.scores_out != nullptr) a.scores_out[row * a.P + p0 + lane] = sc;
-    }
-    if (a.tile_mm != nullptr) tile_key_range(a, row, p0, lane < np, sc);
-  }
-}
-
-// Scores of one tile for D = DFIX and at most 4 heads, in two phases:
-// channels [0, DFIX/2) of every page are stored and scored while the loads
-// of channels [DFIX/2, DFIX) are still in flight.  Each accumulator takes
-// its 32-channel chunks in the same order as the one-phase path (c = 0, 1
-// here, then c = 2, 3), so the scores are identical.
-template <typename DT, int DFIX>
-__device__ void score_tile_split(const ScoreArgs& a, int g, int p0, int np_cap, int length, uint8_t* lds) {
-  using S = typename DT::storage;
-  constexpr int es = static_cast<int>(sizeof(S));
-  constexpr int kQuads = DFIX * es / 16;  // 16-byte quads per row
-  constexpr int kHq = kQuads / 2;
-  constexpr int kPerHalf = (2 * kTilePages * kHq + kScoreBlock - 1) / kScoreBlock;
-  constexpr int kChunks = DFIX / 32;
-  constexpr int pitch = DFIX * es + 16;
-  static_assert(4 * DFIX <= kScoreBlock, "one query value per thread");
-  static_assert(kChunks % 2 == 0 && kHq * 16 == (DFIX / 2) * es, "channel halves are whole chunks and quads");
-  const int tid = static_cast<int>(threadIdx.x);
-  const S* mn = static_cast<const S*>(a.pmin) + g * a.group_stride + static_cast<int64_t>(p0) * DFIX;
-  const S* mx = static_cast<const S*>(a.pmax) + g * a.group_stride + static_cast<int64_t>(p0) * DFIX;
-  float* q_lds = reinterpret_cast<float*>(lds + 2 * kTilePages * pitch);
-  // Loads are unconditional (indices clamped into the tile), so they issue
-  // back to back and each store waits only for its own load.
-  const int nq = a.R * DFIX;
-  const float qv0 = a.q[static_cast<int64_t>(g) * a.R * DFIX + (tid < nq ? tid : nq - 1)];
-  const int total_h = 2 * np_cap * kHq;
-  uint4 va[kPerHalf], vb[kPerHalf];
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-#pragma unroll
-    for (int j = 0; j < kPerHalf; ++j) {
-      int i = tid + j * kScoreBlock;
-      i = i < total_h ? i : total_h - 1;
-      const bool which = i >= np_cap * kHq;
-      const int rem = i - (which ? np_cap * kHq : 0);
-      const int page = rem / kHq;
-      const int qd = rem % kHq + h * kHq;
-      const uint4 v = load_stream(reinterpret_cast<const uint4*>(which ? mx : mn) + page * kQuads + qd);
-      if (h == 0) va[j] = v; else vb[j] = v;
-    }
-    // the first half's loads go out first (and so arrive first)
-    __builtin_amdgcn_sched_barrier(0);
-  }
-  auto store_half = [&](int h, const uint4 (&v)[kPerHalf]) {
-#pragma unroll
-    for (int j = 0; j < kPerHalf; ++j) {
-      // clamped like the loads: a thread past the tile stores the last
-      // quad's value to the last quad's place again
-      int i = tid + j * kScoreBlock;
-      i = i < total_h ? i : total_h - 1;
-      const bool which = i >= np_cap * kHq;
-      const int rem = i - (which ? np_cap * kHq : 0);
-      const int page = rem / kHq;
-      const int qd = rem % kHq + h * kHq;
-      *reinterpret_cast<uint4*>(lds + ((which ? kTilePages : 0) + page) * pitch + qd * 16) = v[j];
-    }
-  };
-  // (unconditional, so the query load is not sunk behind the tile loads;
-  // threads past R*D repeat the last value)
-  q_lds[tid < nq ? tid : nq - 1] = qv0;
-  store_half(0, va);
-  const int P = a.lengths != nullptr ? ragged_pages(length, a.sink, a.recent, a.bs, a.P) : a.P;
-  if (p0 >= P) return;  // block-uniform
-  const int np = (P - p0) < kTilePages ? (P - p0) : kTilePages;
-  __syncthreads();
-  const int wave = wave_uniform(tid / kWave);
-  const int lane = lane_id();
-  const int half = wave / 4;
-  const int r = wave % 4;
-  const bool active = r < a.R;
-  const float* qh = q_lds + r * DFIX;
-  const uint8_t* min_row = lds + lane * pitch;
-  const uint8_t* max_row = lds + (kTilePages + lane) * pitch;
-  float acc[16];
-#pragma unroll
-  for (int l = 0; l < 16; ++l) acc[l] = 0.0f;
-  auto chunks = [&](int c_begin, int c_end) {
-#pragma unroll
-    for (int c = c_begin; c < c_end; ++c) {
-#pragma unroll
-      for (int e = 0; e < 2; ++e) {
-        const int d0 = 32 * c + 16 * half + 8 * e;
-        float qv[8], x[8];
-        *reinterpret_cast<float4*>(qv) = *reinterpret_cast<const float4*>(qh + d0);
-        *reinterpret_cast<float4*>(qv + 4) = *reinterpret_cast<const float4*>(qh + d0 + 4);
-        select8(min_row + d0 * es, max_row + d0 * es, qv, x, DT{});
-#pragma unroll
-        for (int i = 0; i < 8; ++i) acc[8 * e + i] = acc[8 * e + i] + x[i] * qv[i];
-      }
-    }
-  };
-  if (active) chunks(0, kChunks / 2);
-  store_half(1, vb);
-  __syncthreads();
-  if (active) chunks(kChunks / 2, kChunks);
-#pragma unroll
-  for (int w = 1; w < 16; w <<= 1) {
-#pragma unroll
-    for (int l = 0; l < 16; l += 2 * w) acc[l] = acc[l] + acc[l + w];
-  }
-  __shared__ float s_half[4][kWave];
-  if (half == 1) s_half[r][lane] = acc[0];
-  __syncthreads();
-  if (half == 0 && active) {
-    const float sc = acc[0] + s_half[r][lane];
-    const int64_t row = static_cast<int64_t>(g) * a.R + r;
     if (lane < np) {
       a.scores[row * a.score_stride + p0 + lane] = sc;
       if (a.scores_out != nullptr) a.scores_out[row * a.P + p0 + lane] = sc;
@@ -468,14 +359,6 @@ __device__ void score_tile(const ScoreArgs& a, int g, int tile, uint8_t* lds) {
     if (p0 >= p_cap) return;  // block-uniform
   }
   const int np_cap = (p_cap - p0) < kTilePages ? (p_cap - p0) : kTilePages;
-  if constexpr (DFIX > 0) {
-    const uintptr_t base = reinterpret_cast<uintptr_t>(static_cast<const S*>(a.pmin) + g * a.group_stride) |
-                           reinterpret_cast<uintptr_t>(static_cast<const S*>(a.pmax) + g * a.group_stride);
-    if (a.R <= 4 && (base % 16) == 0) {
-      score_tile_split<DT, DFIX>(a, g, p0, np_cap, length, lds);
-      return;
-    }
-  }
   const int pitch = a.D * static_cast<int>(sizeof(S)) + 16;  // 16-byte aligned rows, padded
   float* q_lds = reinterpret_cast<float*>(lds + 2 * kTilePages * pitch);
   stage_tile<DT>(a, g, p0, np_cap, lds, pitch, q_lds);
@@ -1146,13 +1029,17 @@ int launch_score(const ScoreArgs& a, hipStream_t stream) {
   // every tile row starts on 16 bytes, and the heads' accumulators fit the registers
   const bool aligned = ((reinterpret_cast<uintptr_t>(a.pmin) | reinterpret_cast<uintptr_t>(a.pmax)) % 16) == 0 &&
                        (a.G == 1 || (a.group_stride * sizeof(typename DT::storage)) % 16 == 0);
-  const bool tile_path = a.D == 128 && a.R > 4 && a.R <= 8 && aligned;
+  const bool tile_path = a.D == 128 && a.R <= 8 && aligned;
   const size_t lds =
       tile_bytes + static_cast<size_t>(a.R) * (tile_path ? kScoreWaves * kWave : a.D) * sizeof(float);
   if (lds > 160 * 1024) return TW_EUNSUPPORTED;  // gfx950: 160 KB of LDS per CU
   void (*kern)(ScoreArgs) = a.D == 128 ? quest_score_kernel<DT, 128> : quest_score_kernel<DT, 0>;
   if (tile_path) {
     switch (a.R) {
+      case 1: kern = quest_score_tile_kernel<DT, 1>; break;
+      case 2: kern = quest_score_tile_kernel<DT, 2>; break;
+      case 3: kern = quest_score_tile_kernel<DT, 3>; break;
+      case 4: kern = quest_score_tile_kernel<DT, 4>; break;
       case 5: kern = quest_score_tile_kernel<DT, 5>; break;
       case 6: kern = quest_score_tile_kernel<DT, 6>; break;
       case 7: kern = quest_score_tile_kernel<DT, 7>; break;

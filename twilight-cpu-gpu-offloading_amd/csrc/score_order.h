@@ -57,7 +57,6 @@ __device__ __forceinline__ void select8(const uint8_t* mn, const uint8_t* mx, co
 // multiply, add).  The accumulators and their adjacent-pair tree are those of
 // the 32-accumulator order: the in-lane tree covers 4, the combine the other 8.
 constexpr int kScoreWaves = 8;
-typedef const __attribute__((address_space(4))) uint32_t* ConstWords;
 
 __device__ __forceinline__ void load4(const uint8_t* p, float (&x)[4], F16) {
   const uint2 w = *reinterpret_cast<const uint2*>(p);
@@ -77,25 +76,42 @@ __device__ __forceinline__ void load4(const uint8_t* p, float (&x)[4], F32) {
   *reinterpret_cast<float4*>(x) = *reinterpret_cast<const float4*>(p);
 }
 
-// Adds 32-channel chunks [C0, C1) of the wavefront's residues to acc for R
-// heads.  qg: the group's q, [R][128].
-template <typename DT, int R, int C0, int C1>
-__device__ __forceinline__ void score_chunks(const uint8_t* min_row, const uint8_t* max_row, int wave, const float* qg,
-                                             float (&acc)[R][4]) {
-  constexpr int es = static_cast<int>(sizeof(typename DT::storage));
-  const ConstWords q = (ConstWords)(reinterpret_cast<uintptr_t>(qg));
+// The queries of two 32-channel chunks from C0 on, at the wavefront's
+// residues, into scalar registers.  qg: the group's q, [R][128].  All loads go
+// out together and ahead of what the wavefront waits for next: one by one at
+// their uses, each is a round trip of its own (scalar loads return out of order,
+// so every use waits for all of them).
+template <int R>
+struct ScoreQ {
+  u32x4 w[2][R];
+  __device__ __forceinline__ void load(const float* qg, int wave, int C0) {
+    typedef const __attribute__((address_space(4))) u32x4* ConstQuads;
+    const ConstQuads q = (ConstQuads)(reinterpret_cast<uintptr_t>(qg));
 #pragma unroll
-  for (int c = C0; c < C1; ++c) {
-    const int d0 = 32 * c + 4 * wave;
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int r = 0; r < R; ++r) w[c][r] = q[r * 32 + 8 * (C0 + c) + wave];
+    __builtin_amdgcn_sched_barrier(0);
+  }
+};
+
+// Adds 32-channel chunks C0 and C0 + 1 of the wavefront's residues to acc for R
+// heads.
+template <typename DT, int R, int C0>
+__device__ __forceinline__ void score_chunks(const uint8_t* min_row, const uint8_t* max_row, int wave,
+                                             const ScoreQ<R>& q, float (&acc)[R][4]) {
+  constexpr int es = static_cast<int>(sizeof(typename DT::storage));
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    const int d0 = 32 * (C0 + c) + 4 * wave;
     float lo[4], hi[4];
     load4(min_row + d0 * es, lo, DT{});
     load4(max_row + d0 * es, hi, DT{});
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      const int at = r * 128 + d0;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const uint32_t qb = q[at + i];
+        const uint32_t qb = q.w[c][r][i];
         const bool up = static_cast<int32_t>(qb) > 0;  // q > 0 on its bits (a NaN's product is a NaN either way)
         acc[r][i] = acc[r][i] + (up ? hi[i] : lo[i]) * __uint_as_float(qb);
       }
