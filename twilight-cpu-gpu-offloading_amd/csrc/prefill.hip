@@ -21,8 +21,8 @@
 // Bound: the matrix cores and, beside them, the vector unit (a score costs a
 // multiply-add, an exponential, a sum, half a conversion and half a maximum: as
 // many issue cycles as its share of the products).  8 KV heads of 4 query heads,
-// bf16: 32768 rows 8.3 ms, 1060 TFLOP/s of the causal half (a library product of
-// 8192^3 reaches 1186 here), against 137 ms for the score tiles in fp32 through
+// bf16: 32768 rows 8.3 ms, 1060 TFLOP/s of the causal half (library products of
+// 8192^3 and 16384^3 reach 1317 and 1587 here), against 137 ms for the score tiles in fp32 through
 // batched products, mask and softmax; 2048 rows 69 us against 1.0 ms.  The
 // matrix cores are busy 53% of that time, at 1.9 GHz under this load.  Two 32-row
 // query tiles a wavefront (half the LDS reads a product, one wavefront a SIMD)
