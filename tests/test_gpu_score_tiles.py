@@ -54,6 +54,18 @@ def test_scores_off_the_16_byte_grid(dev):
     assert torch.equal(a.view(torch.int32), b.view(torch.int32))
 
 
+def test_queries_off_the_16_byte_grid(dev):
+    """Queries that start four bytes into a row of 16: the scalar loads need no more than a word's alignment."""
+    from headinfer import kernels
+
+    for R in (1, 4, 7, 8):
+        q, lo, hi = _operands(3, R, 130, "bf16", 11, dev)
+        odd = torch.empty(q.numel() + 1, dtype=q.dtype, device=dev)[1:].view(q.shape).copy_(q)
+        assert odd.data_ptr() % 16 == 4
+        got = kernels.fused_quest_score(odd, lo, hi)
+        assert np.array_equal(got.cpu().numpy().view(np.uint32), _want(q, lo, hi, "bf16").view(np.uint32)), R
+
+
 @pytest.mark.parametrize("R", [4, 7])
 @pytest.mark.parametrize("G,P", [(4, 200), (9, 1900)])  # 16 and 270 blocks
 def test_ragged_scores_select_the_same_pages(dev, G, P, R):
