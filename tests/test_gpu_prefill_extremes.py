@@ -1,0 +1,79 @@
+"""The prompt attention at the ends of its operands' range, both kernels and
+both types: rows whose first keys weigh nothing, scores of any finite size,
+scales down to the smallest float, values up to the largest bfloat16.
+
+Limit: a row is a convex combination of V rows and its weights and output are
+each rounded once to the 16-bit type, whose unit roundoff is u = 2^-8 (bf16) or
+2^-11 (fp16): |error| <= 2 u max |v|, and 2^-12 max |v| for the fp32 terms."""
+
+from __future__ import annotations
+
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+U = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}
+# one head: blocks of 128 rows; 512 heads of one: 512 and more blocks of 256 rows, the wide kernel
+KERNELS = pytest.mark.parametrize("heads", [1, 512], ids=["narrow", "wide"])
+DTYPES = pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+SCALE = 128 ** -0.5
+
+
+def _randn(shape, dtype, seed):
+    return torch.randn(shape, generator=torch.Generator(device="cuda").manual_seed(seed), device="cuda").to(dtype)
+
+
+def _reference(q, k, v, scale):
+    """Float64, q/k/v [S, 128] of one head."""
+    S = q.shape[0]
+    s = (q.double() @ k.double().T) * scale
+    future = torch.ones((S, S), dtype=torch.bool, device=q.device).triu(1)
+    return torch.softmax(s.masked_fill(future, -math.inf), dim=-1) @ v.double()
+
+
+def _attention(q, k, v, scale, heads):
+    """[S, 128] of one head, computed `heads` times over one KV head: every copy gives the same bits."""
+    from headinfer import kernels
+
+    S = q.shape[0]
+    out = kernels.prefill_attention(q[None, None].expand(1, heads, -1, -1), k[None, None], v[None, None], scale)
+    out = out.view(S, heads, 128)
+    assert torch.equal(out.view(torch.int16), out[:, :1].expand_as(out).contiguous().view(torch.int16))
+    return out[:, 0]
+
+
+def _close(out, ref, v, dtype):
+    assert torch.equal(out.isnan(), ref.isnan())
+    limit = (2 * U[dtype] + 2.0 ** -12) * float(v.double().abs().max())
+    assert float((out.double() - ref).nan_to_num().abs().max()) <= limit
+
+
+@KERNELS
+@DTYPES
+@pytest.mark.parametrize("S,n", [(200, 63), (200, 64), (300, 128), (300, 130), (450, 257)])
+def test_leading_keys_of_minus_infinity(S, n, dtype, heads):
+    """The first n keys score -inf in every row: rows that see another key are finite, the others 0 / 0."""
+    q, k, v = (_randn((S, 128), dtype, seed=i) for i in range(3))
+    q[:, 0] = 1.0
+    k[:n, 0] = -math.inf
+    ref = _reference(q, k, v, SCALE)
+    assert bool(ref[:n].isnan().all()) and bool(ref[n:].isfinite().all())
+    _close(_attention(q, k, v, SCALE, heads), ref, v, dtype)
+
+
+@KERNELS
+def test_leading_keys_past_the_float_range(heads):
+    """bfloat16 products below -3.4e38 in every second row, finite scores in the others of the wavefront."""
+    S, n = 300, 130
+    q, k, v = (_randn((S, 128), torch.bfloat16, seed=i) for i in range(3))
+    q[:, 0] = 0.0
+    q[::2, 0] = 3e38
+    k[:, 0] = 0.0
+    k[:n, 0] = -3e38
+    out, ref = _attention(q, k, v, SCALE, heads), _reference(q, k, v, SCALE)
+    keep = torch.arange(S, device="cuda") % 2 == 1
+    keep[n:] = True
+    _close(out[keep], ref[keep], v, torch.bfloat16)

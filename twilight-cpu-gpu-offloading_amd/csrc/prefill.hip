@@ -105,6 +105,13 @@ __device__ __forceinline__ float both_halves_sum(float x) {
   return __uint_as_float(h[0]) + __uint_as_float(h[1]);
 }
 
+// What the exponents of a row with maximum m are taken against.  A row whose keys so
+// far all score -inf has no maximum yet: against 0 those keys weigh 0 (-inf
+// against -inf is a NaN that would stay in the row's sums).
+__device__ __forceinline__ float exponent_shift(float m, float scale_log2) {
+  return m == -__builtin_inff() ? 0.0f : m * scale_log2;
+}
+
 // Q^T fragments of query row `row`, rotated if the tables are given.
 template <typename DT>
 __device__ __forceinline__ void load_queries(const PrefillArgs& a, int head, int row, int half,
@@ -243,7 +250,7 @@ __global__ __launch_bounds__(4 * kWave, 2) void prefill_attn_kernel(PrefillArgs 
 #pragma unroll
           for (int i = 0; i < 16; ++i) o[c][i] *= f;
       }
-      const float ms = m * a.scale_log2;
+      const float ms = exponent_shift(m, a.scale_log2);
       float sum = 0.0f;
       frag pf[4];
 #pragma unroll
@@ -469,7 +476,7 @@ __global__ __launch_bounds__(kWideThreads, 2) void prefill_attn_wide(PrefillArgs
         // an unmoved maximum keeps its sums (-inf - -inf is not a factor)
         f = m == mn ? 1.0f : __builtin_amdgcn_exp2f((m - mn) * a.scale_log2);
         m = mn;
-        ms = m * a.scale_log2;
+        ms = exponent_shift(m, a.scale_log2);
       } else {
 #pragma unroll
         for (int i = exp_begin(j); i < exp_begin(j + 1); ++i) {
