@@ -77,3 +77,23 @@ def test_leading_keys_past_the_float_range(heads):
     keep = torch.arange(S, device="cuda") % 2 == 1
     keep[n:] = True
     _close(out[keep], ref[keep], v, torch.bfloat16)
+
+
+@KERNELS
+@DTYPES
+@pytest.mark.parametrize("size", [1.0, 100.0, 1000.0, 6000.0, 20000.0, 60000.0])
+@pytest.mark.parametrize("sign", [1.0, -1.0])
+def test_large_scores(size, sign, dtype, heads):
+    """Equal scores of up to 5e10 average their rows; scores that differ by more than the range of the exponential
+    pick one row, wherever in the prompt it is."""
+    S = 300
+    v = _randn((S, 128), dtype, seed=1)
+    q = torch.full((S, 128), size, device="cuda").to(dtype)
+    k = sign * q
+    _close(_attention(q, k, v, SCALE, heads), _reference(q, k, v, SCALE), v, dtype)
+    if size < 1000.0:
+        return
+    # eight key sizes a factor 2^-1 .. 2^-8 apart, in no order
+    k = k * torch.exp2(-1.0 - torch.randint(0, 8, (S, 1), generator=torch.Generator(device="cuda").manual_seed(2),
+                                            device="cuda")).to(dtype)
+    _close(_attention(q, k, v, SCALE, heads), _reference(q, k, v, SCALE), v, dtype)

@@ -105,12 +105,31 @@ __device__ __forceinline__ float both_halves_sum(float x) {
   return __uint_as_float(h[0]) + __uint_as_float(h[1]);
 }
 
-// What the exponents of a row with maximum m are taken against.  A row whose keys so
-// far all score -inf has no maximum yet: against 0 those keys weigh 0 (-inf
-// against -inf is a NaN that would stay in the row's sums).
-__device__ __forceinline__ float exponent_shift(float m, float scale_log2) {
-  return m == -__builtin_inff() ? 0.0f : m * scale_log2;
-}
+// A weight is 2^(x unit - shift) of a score x: unit = scale_log2 and shift =
+// m scale_log2 against the row's maximum m, one multiply-add a score.  The shift
+// is rounded, by up to half a unit in its last place for every key of the row
+// alike; past kNearShift (2^-15 there), where that would in the end be
+// hundreds of powers of two, the scores themselves become (x - m) scale_log2
+// first, 0 for the maximum.
+//
+// A row whose keys so far all score -inf has no maximum yet: against 0 those keys
+// weigh 0 (-inf against -inf is a NaN that would stay in the row's sums).
+constexpr float kNearShift = 1024.0f;
+struct Exponents {
+  float unit, shift;
+  __device__ __forceinline__ Exponents(f32x16 (&sc)[2], float m, float scale_log2)
+      : unit(scale_log2), shift(m * scale_log2) {
+    if (__any(!(fabsf(shift) <= kNearShift))) {  // hardly ever taken
+      const float against = m == -__builtin_inff() ? 0.0f : m;
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) sc[kb][i] = (sc[kb][i] - against) * scale_log2;
+      unit = 1.0f;
+      shift = 0.0f;
+    }
+  }
+};
 
 // Q^T fragments of query row `row`, rotated if the tables are given.
 template <typename DT>
@@ -239,7 +258,7 @@ __global__ __launch_bounds__(4 * kWave, 2) void prefill_attn_kernel(PrefillArgs 
       }
       mx = fmaxf(max3(mx, sc[0][15], sc[1][15]), mx1);
       mx = both_halves_max(mx);
-      if (__any(mx > m + slack)) {
+      if (__any(mx - m > slack)) {
         const float mn = fmaxf(m, mx);
         // an unmoved maximum keeps its sums (-inf - -inf is not a factor)
         const float f = m == mn ? 1.0f : __builtin_amdgcn_exp2f((m - mn) * a.scale_log2);
@@ -250,7 +269,7 @@ __global__ __launch_bounds__(4 * kWave, 2) void prefill_attn_kernel(PrefillArgs 
 #pragma unroll
           for (int i = 0; i < 16; ++i) o[c][i] *= f;
       }
-      const float ms = exponent_shift(m, a.scale_log2);
+      const Exponents ex(sc, m, a.scale_log2);
       float sum = 0.0f;
       frag pf[4];
 #pragma unroll
@@ -259,7 +278,7 @@ __global__ __launch_bounds__(4 * kWave, 2) void prefill_attn_kernel(PrefillArgs 
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
           const float p =
-              __builtin_amdgcn_exp2f(__builtin_fmaf(sc[ks / 2][8 * (ks % 2) + i], a.scale_log2, -ms));
+              __builtin_amdgcn_exp2f(__builtin_fmaf(sc[ks / 2][8 * (ks % 2) + i], ex.unit, -ex.shift));
           sum += p;
           w[i] = Frag<DT>::narrow(p);
         }
@@ -453,7 +472,7 @@ __global__ __launch_bounds__(kWideThreads, 2) void prefill_attn_wide(PrefillArgs
         for (int i = 0; i < 16; ++i)
           if (32 * kb + (i % 4) + 8 * (i / 4) > limit) sc[kb][i] = -__builtin_inff();
     }
-    float mx = -__builtin_inff(), f = 1.0f, ms = 0.0f, sum = 0.0f, p0 = 0.0f;
+    float mx = -__builtin_inff(), f = 1.0f, unit = 0.0f, shift = 0.0f, sum = 0.0f, p0 = 0.0f;
     bool moved = false;
     uint32_t pw[16];
 #pragma unroll
@@ -471,16 +490,17 @@ __global__ __launch_bounds__(kWideThreads, 2) void prefill_attn_wide(PrefillArgs
         for (int i = 4 * j; i < 4 * j + 4; ++i) mx = max3(mx, sc[0][i], sc[1][i]);
       } else if (j == kMaxSteps) {
         mx = both_halves_max(mx);
-        moved = __any(mx > m + slack);
+        moved = __any(mx - m > slack);
         const float mn = moved ? fmaxf(m, mx) : m;
         // an unmoved maximum keeps its sums (-inf - -inf is not a factor)
         f = m == mn ? 1.0f : __builtin_amdgcn_exp2f((m - mn) * a.scale_log2);
         m = mn;
-        ms = exponent_shift(m, a.scale_log2);
+        const Exponents ex(sc, m, a.scale_log2);
+        unit = ex.unit, shift = ex.shift;
       } else {
 #pragma unroll
         for (int i = exp_begin(j); i < exp_begin(j + 1); ++i) {
-          const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[i / 16][i % 16], a.scale_log2, -ms));
+          const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[i / 16][i % 16], unit, -shift));
           sum += p;
           if (i % 2 == 0)
             p0 = p;
