@@ -97,3 +97,26 @@ def test_large_scores(size, sign, dtype, heads):
     k = k * torch.exp2(-1.0 - torch.randint(0, 8, (S, 1), generator=torch.Generator(device="cuda").manual_seed(2),
                                             device="cuda")).to(dtype)
     _close(_attention(q, k, v, SCALE, heads), _reference(q, k, v, SCALE), v, dtype)
+
+
+@KERNELS
+@DTYPES
+@pytest.mark.parametrize("scale", [1e-20, 2.4e-38, 1e-39, 2.0 ** -149])
+def test_tiny_scales(scale, dtype, heads):
+    """Down to the smallest positive float a row is the plain average of what it sees."""
+    q, k, v = (_randn((300, 128), dtype, seed=i) for i in range(3))
+    _close(_attention(q, k, v, scale, heads), _reference(q, k, v, scale), v, dtype)
+
+
+@pytest.mark.parametrize("scale", [2.0 ** -150, 1e-50, 3e38, 1e39])
+def test_scales_outside_the_float_range(scale):
+    """A scale that is not a float, or whose product with log2 e is not, goes to the torch path as a type that the
+    kernels do not take does."""
+    from headinfer import kernels, mp
+
+    q, k, v = (_randn((1, 1, 80, 128), torch.bfloat16, seed=i) for i in range(3))
+    assert not kernels.prefill_attention_fits(q, k, v, scale)
+    out = mp._prefill_attention(q * 1e-15, k * 1e-15, v, scale)
+    odd = torch.zeros((1, 1, 80, 129), dtype=torch.bfloat16, device="cuda")[..., :128].copy_(k * 1e-15)
+    want = mp._prefill_attention(q * 1e-15, odd, v, scale)
+    assert torch.equal(out.isnan(), want.isnan()) and torch.equal(out.nan_to_num(), want.nan_to_num())

@@ -30,6 +30,7 @@
 // a phase, 8.7 ms.
 #pragma clang fp contract(off)
 
+#include <limits>
 #include <type_traits>
 
 #include "rope.h"
@@ -60,6 +61,11 @@ struct PrefillArgs {
   int64_t cos_row, sin_row;
   int S, G, R, tiles;
   float scale_log2;
+  // Raw scores past the running maximum by less than this (8 / scale_log2) are
+  // taken without moving it: their weights stay below 2^8, and the accumulators
+  // are not rescaled on every tile.  Finite for any scale, so that a first maximum,
+  // up from -inf, is always taken.
+  float slack;
 };
 
 template <typename DT>
@@ -218,10 +224,6 @@ __global__ __launch_bounds__(4 * kWave, 2) void prefill_attn_kernel(PrefillArgs 
   for (int c = 0; c < 4; ++c)
 #pragma unroll
     for (int i = 0; i < 16; ++i) o[c][i] = 0.0f;
-  // raw scores past the running maximum by less than this are taken without
-  // moving it: their weights stay below 2^8, and the accumulators are not
-  // rescaled on every tile
-  const float slack = 8.0f / a.scale_log2;
 
   LOAD_TILE(0)
   STORE_TILE(0)
@@ -258,7 +260,7 @@ __global__ __launch_bounds__(4 * kWave, 2) void prefill_attn_kernel(PrefillArgs 
       }
       mx = fmaxf(max3(mx, sc[0][15], sc[1][15]), mx1);
       mx = both_halves_max(mx);
-      if (__any(mx - m > slack)) {
+      if (__any(mx - m > a.slack)) {
         const float mn = fmaxf(m, mx);
         // an unmoved maximum keeps its sums (-inf - -inf is not a factor)
         const float f = m == mn ? 1.0f : __builtin_amdgcn_exp2f((m - mn) * a.scale_log2);
@@ -397,10 +399,6 @@ __global__ __launch_bounds__(kWideThreads, 2) void prefill_attn_wide(PrefillArgs
   for (int c = 0; c < 4; ++c)
 #pragma unroll
     for (int i = 0; i < 16; ++i) o[c][i] = 0.0f;
-  // raw scores past the running maximum by less than this are taken without
-  // moving it: their weights stay below 2^8, and the accumulators are not
-  // rescaled on every tile
-  const float slack = 8.0f / a.scale_log2;
 
   // fragment addresses in the first tile; the tile and the rest of the row index are immediates
   typedef __attribute__((address_space(3))) char* lds_ptr;
@@ -490,7 +488,7 @@ __global__ __launch_bounds__(kWideThreads, 2) void prefill_attn_wide(PrefillArgs
         for (int i = 4 * j; i < 4 * j + 4; ++i) mx = max3(mx, sc[0][i], sc[1][i]);
       } else if (j == kMaxSteps) {
         mx = both_halves_max(mx);
-        moved = __any(mx - m > slack);
+        moved = __any(mx - m > a.slack);
         const float mn = moved ? fmaxf(m, mx) : m;
         // an unmoved maximum keeps its sums (-inf - -inf is not a factor)
         f = m == mn ? 1.0f : __builtin_amdgcn_exp2f((m - mn) * a.scale_log2);
@@ -649,6 +647,7 @@ extern "C" int tw_prefill_attention(const void* q, const void* k, const void* v,
   a.out_row = static_cast<int64_t>(G) * R * D;
   a.S = S, a.G = G, a.R = R;
   a.scale_log2 = softmax_scale * 1.4426950408889634f;
+  a.slack = fminf(8.0f / a.scale_log2, std::numeric_limits<float>::max());
   const hipStream_t s = static_cast<hipStream_t>(stream);
   return dtype == TW_DTYPE_F16 ? launch<F16>(a, s) : launch<BF16>(a, s);
 }

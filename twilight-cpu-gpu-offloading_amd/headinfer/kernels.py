@@ -1807,7 +1807,7 @@ def decode_attention_varlen(
 # ----------------------------------------------------------------- prefill
 def prefill_attention_fits(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: float) -> bool:
     """Whether prefill_attention takes these operands: 16-bit device tensors of one device with head_dim 128, rows
-    of contiguous channels that start on 16 bytes, and a positive scale."""
+    of contiguous channels that start on 16 bytes, and a scale that is a positive float and stays one times log2 e."""
     if q.ndim != 4 or k.ndim != 4 or v.shape != k.shape or q.shape[0] != 1 or k.shape[0] != 1:
         return False
     if q.dtype not in (torch.float16, torch.bfloat16) or k.dtype != q.dtype or v.dtype != q.dtype:
@@ -1817,8 +1817,10 @@ def prefill_attention_fits(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, sc
     _, Hq, S, D = q.shape
     if D != 128 or k.shape[2:] != (S, D) or not 0 < S <= 1 << 24 or k.shape[1] == 0 or Hq % k.shape[1] or Hq == 0:
         return False
-    return scale > 0.0 and all(t.stride(3) == 1 and t.stride(1) % 8 == 0 and t.stride(2) % 8 == 0
-                               and t.data_ptr() % 16 == 0 for t in (q, k, v))
+    if not 2.0 ** -149 <= scale <= torch.finfo(torch.float32).max / 1.4427:
+        return False
+    return all(t.stride(3) == 1 and t.stride(1) % 8 == 0 and t.stride(2) % 8 == 0 and t.data_ptr() % 16 == 0
+               for t in (q, k, v))
 
 
 def rope_tables_fit(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> bool:
