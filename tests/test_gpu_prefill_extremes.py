@@ -120,3 +120,34 @@ def test_scales_outside_the_float_range(scale):
     odd = torch.zeros((1, 1, 80, 129), dtype=torch.bfloat16, device="cuda")[..., :128].copy_(k * 1e-15)
     want = mp._prefill_attention(q * 1e-15, odd, v, scale)
     assert torch.equal(out.isnan(), want.isnan()) and torch.equal(out.nan_to_num(), want.nan_to_num())
+
+
+@KERNELS
+@pytest.mark.parametrize("size", [1e30, 1e36, 1e38])
+@pytest.mark.parametrize("spread", [0.0, 1.0, 8.0])
+def test_large_values(size, spread, heads):
+    """V near the top of bfloat16's range: the weights' sum before the division may exceed 1 by the prompt's length."""
+    S = 600
+    q, k, v = (_randn((S, 128), torch.bfloat16, seed=i) for i in range(3))
+    v = (v.float().clamp(-3, 3) * size).to(torch.bfloat16)
+    out, ref = _attention(q * spread, k, v, SCALE, heads), _reference(q * spread, k, v, SCALE)
+    _close(out, ref, v, torch.bfloat16)
+
+
+@KERNELS
+def test_large_values_beside_ordinary_ones(heads):
+    """A row that sees no large value keeps its precision beside rows that do; infinities and NaN stay where they are."""
+    S = 400
+    q, k, v = (_randn((S, 128), torch.bfloat16, seed=i) for i in range(3))
+    small = _reference(q, k, v, SCALE)
+    v[200:300] = 3e38
+    ref = _reference(q, k, v, SCALE)
+    top = v.clone()
+    v[300, 5] = math.inf
+    v[301, 6] = math.nan
+    out = _attention(q, k, v, SCALE, heads)
+    # (rows 256 .. 300 share a tile of keys with the infinity: 0 times it is a NaN, as in torch's products)
+    _close(out[:192], small[:192], v[:200], torch.bfloat16)
+    _close(out[192:256], ref[192:256], top, torch.bfloat16)
+    assert bool(out[301:, 5].isinf().all()) and bool(out[301:, 6].isnan().all())
+    _close(out[301:, 7:], ref[301:, 7:], top, torch.bfloat16)

@@ -123,8 +123,8 @@ __device__ __forceinline__ float both_halves_sum(float x) {
 constexpr float kNearShift = 1024.0f;
 struct Exponents {
   float unit, shift;
-  __device__ __forceinline__ Exponents(f32x16 (&sc)[2], float m, float scale_log2)
-      : unit(scale_log2), shift(m * scale_log2) {
+  __device__ __forceinline__ Exponents(f32x16 (&sc)[2], float m, float scale_log2, float drop)
+      : unit(scale_log2), shift(m * scale_log2 + drop) {
     if (__any(!(fabsf(shift) <= kNearShift))) {  // hardly ever taken
       const float against = m == -__builtin_inff() ? 0.0f : m;
 #pragma unroll
@@ -132,10 +132,17 @@ struct Exponents {
 #pragma unroll
         for (int i = 0; i < 16; ++i) sc[kb][i] = (sc[kb][i] - against) * scale_log2;
       unit = 1.0f;
-      shift = 0.0f;
+      shift = drop;
     }
   }
 };
+
+// The powers of two by which a block's second pass lowers its weights.  A weight is
+// below 2^8 and their sum below 2^8 S, so V past the largest float over that may
+// leave the accumulators' range though the row, their quotient, is in it; lowered,
+// |o| stays below half the largest |v|.  (Lowered in every pass, the smallest V
+// would fall below the range instead.  fp16 values have no such size.)
+__device__ __forceinline__ float second_pass_drop(int S) { return static_cast<float>(9 + 32 - __clz(S)); }
 
 // Q^T fragments of query row `row`, rotated if the tables are given.
 template <typename DT>
@@ -170,24 +177,43 @@ __device__ __forceinline__ void load_queries(const PrefillArgs& a, int head, int
   }
 }
 
-// A block of 4 wavefronts, each taking a tile's scores, weights and values in
-// turn; two blocks share a CU and drift apart.
+// Stores the lane's half of its row, o / l, if `store`; whether it held an infinity or a NaN.
 template <typename DT>
-__global__ __launch_bounds__(4 * kWave, 2) void prefill_attn_kernel(PrefillArgs a) {
+__device__ __forceinline__ bool store_output(const PrefillArgs& a, int row, int head, int half, bool store,
+                                             const f32x16 (&o)[4], float l) {
+  const float inv = 1.0f / both_halves_sum(l);
+  if (!store) return false;
+  float bad = 0.0f;
+  uint16_t* p = a.out + static_cast<int64_t>(row) * a.out_row + head * kHead + 4 * half;
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      typename Frag<DT>::quad w;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float x = o[c][4 * i + j] * inv;
+        bad = __builtin_fmaf(x, 0.0f, bad);
+        w[j] = Frag<DT>::narrow(x);
+      }
+      *reinterpret_cast<typename Frag<DT>::quad*>(p + 32 * c + 8 * i) = w;
+    }
+  return bad != 0.0f;  // a NaN
+}
+
+// Query rows q_block .. + 32 NW - 1 of a head by a block of NW wavefronts, each
+// taking a tile's scores, weights and values in turn.  Stores the lanes' rows with
+// `store`, weights lowered by 2^drop; whether the lane's held an infinity or a NaN.
+template <typename DT, int NW>
+__device__ __forceinline__ bool attend(const PrefillArgs& a, u32x4* s_tiles, int g, int head, int q_block, bool store,
+                                       float drop) {
   typedef typename Frag<DT>::type frag;
-  constexpr int NW = 4;
   constexpr int kLoads = kKeys * kRowUnits / (NW * kWave);  // 16-byte units a thread stages, for K and for V
-  __shared__ u32x4 s_k[2][kKeys * kRowUnits];
-  __shared__ u32x4 s_v[2][kKeys * kRowUnits];
+  u32x4* const s_k = s_tiles;  // tiles of even and odd index
+  u32x4* const s_v = s_tiles + 2 * kKeys * kRowUnits;
 
   const int tid = threadIdx.x, lane = tid % kWave, wave = wave_uniform(tid / kWave);
   const int col = lane % 32, half = lane / 32;
-  // group-minor, the longest query tiles first
-  const int g = blockIdx.x % a.G;
-  const int rest = blockIdx.x / a.G;
-  const int head = g * a.R + rest % a.R;
-  const int qt = a.tiles - 1 - rest / a.R;
-  const int q_block = qt * NW * kQ;
   const int q0 = q_block + wave * kQ;
   const int S = a.S;
 
@@ -214,8 +240,8 @@ __global__ __launch_bounds__(4 * kWave, 2) void prefill_attn_kernel(PrefillArgs 
 #define STORE_TILE(b)                                                                                      \
   _Pragma("unroll") for (int i = 0; i < kLoads; ++i) {                                                     \
     const int at = slot(st_row + i * (kKeys / kLoads), st_unit);                                           \
-    s_k[b][at] = rk[i];                                                                                    \
-    s_v[b][at] = rv[i];                                                                                    \
+    s_k[(b) * kKeys * kRowUnits + at] = rk[i];                                                             \
+    s_v[(b) * kKeys * kRowUnits + at] = rv[i];                                                             \
   }
 
   f32x16 o[4];
@@ -240,7 +266,7 @@ __global__ __launch_bounds__(4 * kWave, 2) void prefill_attn_kernel(PrefillArgs 
         for (int i = 0; i < 16; ++i) sc[kb][i] = 0.0f;
 #pragma unroll
         for (int s = 0; s < 8; ++s) {
-          const frag kf = __builtin_bit_cast(frag, s_k[b][slot(32 * kb + col, 2 * s + half)]);
+          const frag kf = __builtin_bit_cast(frag, s_k[b * kKeys * kRowUnits + slot(32 * kb + col, 2 * s + half)]);
           sc[kb] = Frag<DT>::mfma(kf, qf[s], sc[kb]);
         }
       }
@@ -271,7 +297,7 @@ __global__ __launch_bounds__(4 * kWave, 2) void prefill_attn_kernel(PrefillArgs 
 #pragma unroll
           for (int i = 0; i < 16; ++i) o[c][i] *= f;
       }
-      const Exponents ex(sc, m, a.scale_log2);
+      const Exponents ex(sc, m, a.scale_log2, drop);
       float sum = 0.0f;
       frag pf[4];
 #pragma unroll
@@ -298,7 +324,7 @@ __global__ __launch_bounds__(4 * kWave, 2) void prefill_attn_kernel(PrefillArgs 
 #pragma unroll
           for (int h = 0; h < 2; ++h) {
             const int r = 16 * ks + 8 * h + vrow, ch = 32 * c + vch;
-            const uint2* p = reinterpret_cast<const uint2*>(&s_v[b][slot(r, ch / 8)]) + (ch % 8) / 4;
+            const uint2* p = reinterpret_cast<const uint2*>(&s_v[b * kKeys * kRowUnits + slot(r, ch / 8)]) + (ch % 8) / 4;
             const s16x4 x = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
                 (__attribute__((address_space(3))) s16x4*)(reinterpret_cast<uintptr_t>(p)));
 #pragma unroll
@@ -314,19 +340,23 @@ __global__ __launch_bounds__(4 * kWave, 2) void prefill_attn_kernel(PrefillArgs 
 #undef LOAD_TILE
 #undef STORE_TILE
 
-  const float inv = 1.0f / both_halves_sum(l);
-  if (row < S) {
-    uint16_t* p = a.out + static_cast<int64_t>(row) * a.out_row + head * kHead + 4 * half;
-#pragma unroll
-    for (int c = 0; c < 4; ++c)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        typename Frag<DT>::quad w;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) w[j] = Frag<DT>::narrow(o[c][4 * i + j] * inv);
-        *reinterpret_cast<typename Frag<DT>::quad*>(p + 32 * c + 8 * i) = w;
-      }
-  }
+  return store_output<DT>(a, row, head, half, store, o, l);
+}
+
+// Blocks of 4 wavefronts; two blocks share a CU and drift apart.
+template <typename DT>
+__global__ __launch_bounds__(4 * kWave, 2) void prefill_attn_kernel(PrefillArgs a) {
+  constexpr int NW = 4;
+  __shared__ u32x4 s_tiles[4 * kKeys * kRowUnits];
+  // group-minor, the longest query tiles first
+  const int g = blockIdx.x % a.G;
+  const int rest = blockIdx.x / a.G;
+  const int head = g * a.R + rest % a.R;
+  const int q_block = (a.tiles - 1 - rest / a.R) * NW * kQ;
+  const int row = q_block + static_cast<int>(threadIdx.x) / kWave * kQ + static_cast<int>(threadIdx.x) % kQ;
+  const bool over = attend<DT, NW>(a, s_tiles, g, head, q_block, row < a.S, 0.0f);
+  if constexpr (std::is_same_v<DT, BF16>)
+    if (__syncthreads_or(over)) attend<DT, NW>(a, s_tiles, g, head, q_block, over, second_pass_drop(a.S));
 }
 
 // Blocks of 8 wavefronts, with the three streams of neighbouring tiles
@@ -493,7 +523,7 @@ __global__ __launch_bounds__(kWideThreads, 2) void prefill_attn_wide(PrefillArgs
         // an unmoved maximum keeps its sums (-inf - -inf is not a factor)
         f = m == mn ? 1.0f : __builtin_amdgcn_exp2f((m - mn) * a.scale_log2);
         m = mn;
-        const Exponents ex(sc, m, a.scale_log2);
+        const Exponents ex(sc, m, a.scale_log2, 0.0f);
         unit = ex.unit, shift = ex.shift;
       } else {
 #pragma unroll
@@ -578,19 +608,9 @@ __global__ __launch_bounds__(kWideThreads, 2) void prefill_attn_wide(PrefillArgs
     __syncthreads();
   }
 
-  const float inv = 1.0f / both_halves_sum(l);
-  if (row < S) {
-    uint16_t* p = a.out + static_cast<int64_t>(row) * a.out_row + head * kHead + 4 * half;
-#pragma unroll
-    for (int c = 0; c < 4; ++c)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        typename Frag<DT>::quad w;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) w[j] = Frag<DT>::narrow(o[c][4 * i + j] * inv);
-        *reinterpret_cast<typename Frag<DT>::quad*>(p + 32 * c + 8 * i) = w;
-      }
-  }
+  const bool over = store_output<DT>(a, row, head, half, row < S, o, l);
+  if constexpr (std::is_same_v<DT, BF16>)
+    if (__syncthreads_or(over)) attend<DT, kWideWaves>(a, s_tiles, g, head, q_block, over, second_pass_drop(S));
 }
 
 constexpr int kWideBlocks = 512;
