@@ -101,3 +101,22 @@ def test_resident_window_sizes(sink, recent, ring):
     assert v.win_state.data_ptr() == res.win_state[2].data_ptr() and v.ring == ring
     plain = ResidentPages(6, 4, 10, 128, torch.bfloat16, torch.device("cpu"))
     assert plain.win_k is None and plain.view(0, 2).win_state is None
+
+
+def test_sequential_state_preview_of_a_run():
+    """A run of entries is refused as appending them in turn would be, with nothing applied."""
+    st = SequentialCacheState(3, 5)
+    assert st.preview_run(0, 3, 4) == [(0, 4)] * 3 and st.preview_run(0, 0, 4) == []
+    for first, count, n in ((1, 1, 4), (0, 4, 2), (0, 3, 0), (0, 1, 6)):
+        with pytest.raises((ValueError, RuntimeError)) as got:
+            st.preview_run(first, count, n)
+        trial = SequentialCacheState(3, 5)
+        with pytest.raises(type(got.value)) as want:
+            for e in range(first, first + count):
+                trial.advance(e, n)
+        assert str(got.value) == str(want.value)
+    assert st.logical_lengths == [0, 0, 0] and st.expected_next_entry == 0
+    st.advance(0, 2)
+    assert st.preview_run(1, 2, 3) == [(0, 3)] * 2
+    with pytest.raises(ValueError):
+        st.preview_run(1, 3, 3)

@@ -184,7 +184,7 @@ def _fused_prompt(cache: Any, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     nothing asks for a derivative and every operand is of the form those kernels read."""
     return (_is_headinfer_cache(cache) and hasattr(cache, "prompt_layer_fits")
             and not _derivative_wanted(q, k, v, cos, sin) and kernels.prefill_attention_fits(q, k, v, scale)
-            and kernels.rope_tables_fit(q, cos, sin) and cache.prompt_layer_fits(k, v, cos, sin))
+            and cache.prompt_layer_fits(k, v, cos, sin))  # (tables that rotate k rotate q)
 
 
 def _fast_forward(self, hidden_states: torch.Tensor, position_embeddings=None, attention_mask=None,

@@ -361,36 +361,48 @@ class QuestTopKOffloadedCache(_CacheBase):
     def update_prompt_layer(self, entry0: int, key_states: torch.Tensor, value_states: torch.Tensor,
                             cos: torch.Tensor, sin: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
         """The prefill `update` of entries [entry0, entry0 + G) in one launch, for K/V [1, G, S, D] with K before its
-        rotary embedding (prompt_layer_fits): rotation, slab write and metadata.  Returns the rotated K and V."""
+        rotary embedding (prompt_layer_fits): rotation, slab write and metadata.  Returns the rotated K and V.  A
+        call that is refused leaves the cache as it was."""
         _, G, S, D = key_states.shape
-        for e in range(entry0, entry0 + G):
-            self._advance_prompt(e, S)
-        pages = self._allocate_metadata(S)
+        for old_length, _ in self._bookkeeping.preview_run(entry0, G, S):
+            self._check_prompt(old_length, S)
         host = self.kv_residency != "hbm"
         if host:
             K, V = torch.empty((2, G, S, D), dtype=self.dtype, device=self.device)
         else:
             K, V = self._key_cache[entry0:entry0 + G, :S], self._value_cache[entry0:entry0 + G, :S]
+        first = self._page_min is None
+        pages = self._allocate_metadata(S)
         assert self._page_min is not None and self._page_max is not None
-        kernels.prompt_kv(key_states, value_states, cos, sin, K, V, sink=self.sink_tokens, block_size=self.block_size,
-                          page_min=self._page_min[entry0:entry0 + G] if pages else None,
-                          page_max=self._page_max[entry0:entry0 + G] if pages else None,
-                          **self._int4_rows(entry0, G))
-        if host:
-            for g in range(G):
+        try:
+            kernels.prompt_kv(key_states, value_states, cos, sin, K, V, sink=self.sink_tokens,
+                              block_size=self.block_size,
+                              page_min=self._page_min[entry0:entry0 + G] if pages else None,
+                              page_max=self._page_max[entry0:entry0 + G] if pages else None,
+                              **self._int4_rows(entry0, G))
+        except Exception:  # operands that it refuses
+            if first:
+                self._page_min = self._page_max = None
+            raise
+        for g in range(G):
+            if host:
                 self._write_prompt(entry0 + g, K[None, g:g + 1], V[None, g:g + 1], 0, S)
+            self._advance_prompt(entry0 + g, S)
         return K[None], V[None]
 
     def _advance_prompt(self, entry: int, length: int) -> Tuple[int, int]:
-        """The bookkeeping of one entry's prompt (the refusals of quest_offload_cache.py:513-537)."""
+        """The bookkeeping of one entry's prompt."""
         old_length, new_length = self._advance_entry(entry, length)
+        self._check_prompt(old_length, length)
+        self._prompt_length = length
+        return old_length, new_length
+
+    def _check_prompt(self, old_length: int, length: int) -> None:
+        """The refusals of quest_offload_cache.py:513-537 that the bookkeeping does not have."""
         if old_length != 0:
             raise ValueError("chunked/multiple prefill updates are unsupported")
-        if self._prompt_length is None:
-            self._prompt_length = length
-        elif self._prompt_length != length:
+        if self._prompt_length not in (None, length):
             raise RuntimeError("cache entries received unequal prompt lengths")
-        return old_length, new_length
 
     def _advance_entry(self, entry: int, length: int) -> Tuple[int, int]:
         lengths = self._bookkeeping.advance(entry, length)

@@ -81,9 +81,18 @@ class SequentialCacheState:
 
     def preview(self, entry_idx: int, append_length: int) -> tuple[int, int]:
         """(old_length, new_length) of an append, validated but not applied."""
-        if entry_idx != self.expected_next_entry:
+        return self._preview(entry_idx, self.expected_next_entry, append_length)
+
+    def preview_run(self, first_entry: int, count: int, append_length: int) -> list[tuple[int, int]]:
+        """preview of appends to `count` entries in turn."""
+        expected = [self.expected_next_entry, *((e + 1) % self.num_entries
+                                                for e in range(first_entry, first_entry + count - 1))]
+        return [self._preview(first_entry + i, expected[i], append_length) for i in range(count)]
+
+    def _preview(self, entry_idx: int, expected: int, append_length: int) -> tuple[int, int]:
+        if entry_idx != expected:
             raise ValueError("strict sequential head-wise update violated: "
-                             f"expected {self.expected_next_entry}, got {entry_idx}")
+                             f"expected {expected}, got {entry_idx}")
         if append_length <= 0:
             raise ValueError("append_length must be positive")
         old = self.logical_lengths[entry_idx]
