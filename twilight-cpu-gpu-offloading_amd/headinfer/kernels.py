@@ -1819,15 +1819,24 @@ def prefill_attention_fits(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, sc
         return False
     if not 2.0 ** -149 <= scale <= torch.finfo(torch.float32).max / 1.4427:
         return False
-    return all(t.stride(3) == 1 and t.stride(1) % 8 == 0 and t.stride(2) % 8 == 0 and t.data_ptr() % 16 == 0
-               for t in (q, k, v))
+    for t in (q, k, v):
+        _, head, row, channel = t.stride()
+        if channel != 1 or head % 8 or row % 8 or t.data_ptr() % 16:
+            return False
+    return True
 
 
 def rope_tables_fit(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> bool:
     """Whether the prompt kernels can rotate x [1, H, S, 128] by cos/sin: [1, S, 128] tables of x's type and device,
     rows of contiguous channels that start on 16 bytes."""
-    return all(t.shape == (1, x.shape[2], x.shape[3]) and t.dtype == x.dtype and t.device == x.device
-               and t.stride(2) == 1 and t.stride(1) % 8 == 0 and t.data_ptr() % 16 == 0 for t in (cos, sin))
+    shape = (1, x.shape[2], x.shape[3])
+    for t in (cos, sin):
+        if t.shape != shape or t.dtype != x.dtype or t.device != x.device:
+            return False
+        _, row, channel = t.stride()
+        if channel != 1 or row % 8 or t.data_ptr() % 16:
+            return False
+    return True
 
 
 def prefill_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: float,

@@ -56,8 +56,31 @@ class _CacheBase(_HFCache):  # type: ignore[misc, valid-type]
             super().__init__()
 
 
-# The per-entry prompt methods that update_prompt_layer stands in for.
-_PROMPT_HOOKS = frozenset({"update", "_build_metadata", "_write_prompt"})
+# The per-entry prompt methods that update_prompt_layer stands in for, as the
+# package's own classes define them.
+_PROMPT_METHODS = ("update", "_build_metadata", "_write_prompt")
+_OWN_PROMPT_METHODS: Dict[type, Dict[str, Any]] = {}
+
+
+def _owns_prompt_methods(cls: type) -> type:
+    """Class decorator: notes the per-entry prompt methods that cls itself defines."""
+    _OWN_PROMPT_METHODS[cls] = {n: vars(cls)[n] for n in _PROMPT_METHODS if n in vars(cls)}
+    return cls
+
+
+def _prompt_methods_replaced(cache: "QuestTopKOffloadedCache") -> bool:
+    """Whether a subclass, an assignment to one of the package's classes or one to the instance replaces a per-entry
+    prompt method."""
+    if not vars(cache).keys().isdisjoint(_PROMPT_METHODS):
+        return True
+    for cls in type(cache).__mro__:
+        has, own = vars(cls), _OWN_PROMPT_METHODS.get(cls, {})
+        for name in _PROMPT_METHODS:
+            if has.get(name) is not own.get(name):
+                return True
+        if cls is QuestTopKOffloadedCache:  # it calls no update of its bases
+            return False
+    return True
 
 
 def _window(length: int, sink: int, recent: int) -> tuple[int, int, int]:
@@ -67,6 +90,7 @@ def _window(length: int, sink: int, recent: int) -> tuple[int, int, int]:
     return sink_end, recent_start, max(0, recent_start - sink_end)
 
 
+@_owns_prompt_methods
 class QuestTopKOffloadedCache(_CacheBase):
     """Slab-backed KV cache with per-query-head Quest top-k page selection."""
 
@@ -350,9 +374,9 @@ class QuestTopKOffloadedCache(_CacheBase):
     def prompt_layer_fits(self, key_states: torch.Tensor, value_states: torch.Tensor, cos: torch.Tensor,
                           sin: torch.Tensor) -> bool:
         """Whether update_prompt_layer takes this layer: 16-bit K/V of the cache's type on its device, 128 channels,
-        16-row pages, tables that rotate them -- and per-entry methods that no subclass or instance replaces."""
-        own = type(self).__module__.startswith(__package__ + ".")
-        return (own and not _PROMPT_HOOKS & vars(self).keys() and key_states.shape[2] > 1
+        16-row pages, tables that rotate them -- and per-entry methods that no subclass, class or instance
+        replaces."""
+        return (not _prompt_methods_replaced(self) and key_states.shape[2] > 1
                 and key_states.dtype == self.dtype and key_states.device == self.device and self.block_size == 16
                 and key_states.shape[3] == self.geometry.head_dim == 128
                 and kernels.prefill_attention_fits(key_states, key_states, value_states, 1.0)

@@ -42,7 +42,7 @@ from typing import Any, Dict, Optional, Sequence
 import torch
 
 from . import kernels
-from .quest_offload_cache import QuestTopKOffloadedCache, _window
+from .quest_offload_cache import QuestTopKOffloadedCache, _owns_prompt_methods, _window
 
 __all__ = [
     "affine_int4_pack",
@@ -140,6 +140,7 @@ def matched_budget_counts_tensor(desired: torch.Tensor, target_total: int, capac
 
 
 # ------------------------------------------------------------------- cache
+@_owns_prompt_methods
 class TwilightMatchedBudgetOffloadedCache(QuestTopKOffloadedCache):
     """Quest B0 + INT4 QK + top-p with matched or dynamic budgets."""
 
