@@ -85,7 +85,8 @@ template <int R>
 struct ScoreQ {
   u32x4 w[2][R];
   __device__ __forceinline__ void load(const float* qg, int wave, int C0) {
-    typedef const __attribute__((address_space(4))) u32x4* ConstQuads;
+    typedef uint32_t WordQuad __attribute__((ext_vector_type(4), aligned(4)));  // queries start on any word
+    typedef const __attribute__((address_space(4))) WordQuad* ConstQuads;
     const ConstQuads q = (ConstQuads)(reinterpret_cast<uintptr_t>(qg));
 #pragma unroll
     for (int c = 0; c < 2; ++c)
