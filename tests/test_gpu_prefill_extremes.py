@@ -1,10 +1,12 @@
 """The prompt attention at the ends of its operands' range, both kernels and
 both types: rows whose first keys weigh nothing, scores of any finite size,
-scales down to the smallest float, values up to the largest bfloat16.
+scales down to the smallest float, values up to the largest bfloat16, long rows
+and row strides past the wide kernel's offsets.
 
 Limit: a row is a convex combination of V rows and its weights and output are
 each rounded once to the 16-bit type, whose unit roundoff is u = 2^-8 (bf16) or
-2^-11 (fp16): |error| <= 2 u max |v|, and 2^-12 max |v| for the fp32 terms."""
+2^-11 (fp16): |error| <= 2 u max |v|, and 2^-12 max |v| for the fp32 terms and
+fp16's weights below 2^-14 (at most 2^-25 each, 600 rows)."""
 
 from __future__ import annotations
 
@@ -151,3 +153,42 @@ def test_large_values_beside_ordinary_ones(heads):
     _close(out[192:256], ref[192:256], top, torch.bfloat16)
     assert bool(out[301:, 5].isinf().all()) and bool(out[301:, 6].isnan().all())
     _close(out[301:, 7:], ref[301:, 7:], top, torch.bfloat16)
+
+
+@KERNELS
+@DTYPES
+def test_row_strides_on_both_sides_of_the_wide_offsets(dtype, heads):
+    """K/V rows up to 2^24 elements apart go to the wide kernel, rows further apart to the other: the same row by row."""
+    from headinfer import kernels
+
+    S, far = 20, 1 << 24
+    q, k, v = (_randn((S, 128), dtype, seed=i) for i in range(3))
+    ref = _reference(q, k, v, SCALE)
+    flat = torch.empty((S - 1) * (far + 8) + 256, dtype=dtype, device="cuda")
+    for stride in (far, far + 8):
+        both = flat.as_strided((2, S, 128), (128, stride, 1))
+        both[0], both[1] = k, v
+        for kk, vv in ((both[0], v), (k, both[1]), (both[0], both[1])):
+            assert kernels.prefill_attention_fits(q[None, None], kk[None, None], vv[None, None], SCALE)
+            _close(_attention(q, kk, vv, SCALE, heads), ref, v, dtype)
+
+
+@DTYPES
+@pytest.mark.parametrize("heads", [1, 8], ids=["narrow", "wide"])  # 157 blocks of 128 rows, 632 of 256
+@pytest.mark.parametrize("spread", [0.1, 3.0])
+def test_long_rows(spread, dtype, heads):
+    """20000 rows: the sums are chains of at most S / 2 fp32 additions, 2^-24 each, 2^-10 max |v| in all; fp16 weights
+    below 2^-14 add S 2^-25."""
+    S = 20000
+    q, k, v = (_randn((S, 128), dtype, seed=i) for i in range(3))
+    q, v = q * spread, v + 1.0
+    out = _attention(q, k, v, SCALE, heads)
+    rows = torch.cat([torch.arange(0, S, 997, device="cuda"), torch.arange(S - 40, S, device="cuda")])
+    s = (q[rows].double() @ k.double().T) * SCALE
+    s.masked_fill_(torch.arange(S, device="cuda")[None] > rows[:, None], -math.inf)
+    ref = torch.softmax(s, dim=-1) @ v.double()
+    limit = (2 * U[dtype] + 2.0 ** -10 + (S * 2.0 ** -25 if dtype == torch.float16 else 0.0)) * float(v.abs().max())
+    assert float((out[rows].double() - ref).abs().max()) <= limit
+    # 2-norm: two independent roundings, each uniform within +- u / m of the value for a mantissa m in [1, 2), an rms
+    # of u / sqrt(6)
+    assert float((out[rows].double() - ref).norm() / ref.norm()) <= 0.6 * U[dtype]

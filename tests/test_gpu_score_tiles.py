@@ -66,7 +66,7 @@ def test_queries_off_the_16_byte_grid(dev):
         assert np.array_equal(got.cpu().numpy().view(np.uint32), _want(q, lo, hi, "bf16").view(np.uint32)), R
 
 
-@pytest.mark.parametrize("R", [4, 7])
+@pytest.mark.parametrize("R", [4, 7, 8])  # (8: some queries outside the scalar registers)
 @pytest.mark.parametrize("G,P", [(4, 200), (9, 1900)])  # 16 and 270 blocks
 def test_ragged_scores_select_the_same_pages(dev, G, P, R):
     from headinfer import kernels
