@@ -143,6 +143,12 @@ struct Exponents {
 // |o| stays below half the largest |v|.  (Lowered in every pass, the smallest V
 // would fall below the range instead.  fp16 values have no such size.)
 __device__ __forceinline__ float second_pass_drop(int S) { return static_cast<float>(9 + 32 - __clz(S)); }
+// Whether some wavefront of the block has `over`; flag: a word of LDS, 0 since the block's start.
+__device__ __forceinline__ bool block_any(bool over, int* flag) {
+  if (__any(over) && lane_id() == 0) *flag = 1;
+  __syncthreads();
+  return *flag != 0;
+}
 
 // Q^T fragments of query row `row`, rotated if the tables are given.
 template <typename DT>
@@ -177,13 +183,13 @@ __device__ __forceinline__ void load_queries(const PrefillArgs& a, int head, int
   }
 }
 
-// Stores the lane's half of its row, o / l, if `store`; whether it held an infinity or a NaN.
+// Stores the lane's half of its row, o / l, if `store`; whether it held an infinity or a NaN (bf16 only).
 template <typename DT>
 __device__ __forceinline__ bool store_output(const PrefillArgs& a, int row, int head, int half, bool store,
                                              const f32x16 (&o)[4], float l) {
   const float inv = 1.0f / both_halves_sum(l);
   if (!store) return false;
-  float bad = 0.0f;
+  float bad[4] = {0.0f, 0.0f, 0.0f, 0.0f};  // four chains of sums of 0 x
   uint16_t* p = a.out + static_cast<int64_t>(row) * a.out_row + head * kHead + 4 * half;
 #pragma unroll
   for (int c = 0; c < 4; ++c)
@@ -193,18 +199,18 @@ __device__ __forceinline__ bool store_output(const PrefillArgs& a, int row, int 
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const float x = o[c][4 * i + j] * inv;
-        bad = __builtin_fmaf(x, 0.0f, bad);
+        if constexpr (std::is_same_v<DT, BF16>) bad[j] = __builtin_fmaf(x, 0.0f, bad[j]);
         w[j] = Frag<DT>::narrow(x);
       }
       *reinterpret_cast<typename Frag<DT>::quad*>(p + 32 * c + 8 * i) = w;
     }
-  return bad != 0.0f;  // a NaN
+  return (bad[0] + bad[1]) + (bad[2] + bad[3]) != 0.0f;  // a NaN
 }
 
 // Query rows q_block .. + 32 NW - 1 of a head by a block of NW wavefronts, each
 // taking a tile's scores, weights and values in turn.  Stores the lanes' rows with
 // `store`, weights lowered by 2^drop; whether the lane's held an infinity or a NaN.
-template <typename DT, int NW>
+template <typename DT, int NW, bool AGAIN>
 __device__ __forceinline__ bool attend(const PrefillArgs& a, u32x4* s_tiles, int g, int head, int q_block, bool store,
                                        float drop) {
   typedef typename Frag<DT>::type frag;
@@ -212,7 +218,9 @@ __device__ __forceinline__ bool attend(const PrefillArgs& a, u32x4* s_tiles, int
   u32x4* const s_k = s_tiles;  // tiles of even and odd index
   u32x4* const s_v = s_tiles + 2 * kKeys * kRowUnits;
 
-  const int tid = threadIdx.x, lane = tid % kWave, wave = wave_uniform(tid / kWave);
+  int tid = threadIdx.x;
+  if constexpr (AGAIN) asm volatile("" : "+v"(tid));  // a second pass forms its addresses anew: kept over the first, they spill
+  const int lane = tid % kWave, wave = wave_uniform(tid / kWave);
   const int col = lane % 32, half = lane / 32;
   const int q0 = q_block + wave * kQ;
   const int S = a.S;
@@ -348,15 +356,17 @@ template <typename DT>
 __global__ __launch_bounds__(4 * kWave, 2) void prefill_attn_kernel(PrefillArgs a) {
   constexpr int NW = 4;
   __shared__ u32x4 s_tiles[4 * kKeys * kRowUnits];
+  __shared__ int s_over;
+  if (threadIdx.x == 0) s_over = 0;  // (ahead of the first of many barriers)
   // group-minor, the longest query tiles first
   const int g = blockIdx.x % a.G;
   const int rest = blockIdx.x / a.G;
   const int head = g * a.R + rest % a.R;
   const int q_block = (a.tiles - 1 - rest / a.R) * NW * kQ;
   const int row = q_block + static_cast<int>(threadIdx.x) / kWave * kQ + static_cast<int>(threadIdx.x) % kQ;
-  const bool over = attend<DT, NW>(a, s_tiles, g, head, q_block, row < a.S, 0.0f);
+  const bool over = attend<DT, NW, false>(a, s_tiles, g, head, q_block, row < a.S, 0.0f);
   if constexpr (std::is_same_v<DT, BF16>)
-    if (__syncthreads_or(over)) attend<DT, NW>(a, s_tiles, g, head, q_block, over, second_pass_drop(a.S));
+    if (block_any(over, &s_over)) attend<DT, NW, true>(a, s_tiles, g, head, q_block, over, second_pass_drop(a.S));
 }
 
 // Blocks of 8 wavefronts, with the three streams of neighbouring tiles
@@ -369,6 +379,8 @@ template <typename DT>
 __global__ __launch_bounds__(kWideThreads, 2) void prefill_attn_wide(PrefillArgs a) {
   typedef typename Frag<DT>::type frag;
   __shared__ u32x4 s_tiles[4 * kKeys * kRowUnits];  // K tiles of even and odd index, then V's
+  __shared__ int s_over;
+  if (threadIdx.x == 0) s_over = 0;  // (ahead of the first of many barriers)
 
   const int tid = threadIdx.x, lane = tid % kWave, wave = wave_uniform(tid / kWave);
   const int col = lane % 32, half = lane / 32;
@@ -422,8 +434,7 @@ __global__ __launch_bounds__(kWideThreads, 2) void prefill_attn_wide(PrefillArgs
 
   f32x16 o[4], sc[2];
   frag p_even[4], p_odd[4];
-  f32x16 zero = {0.0f};
-  asm volatile("" : "+v"(zero));  // kept in registers: the first product of every chain adds to it
+  const f32x16 zero = {0.0f};  // the first product of every chain adds to it (as an operand, in no register)
   float m = -__builtin_inff(), l = 0.0f;
 #pragma unroll
   for (int c = 0; c < 4; ++c)
@@ -610,7 +621,7 @@ __global__ __launch_bounds__(kWideThreads, 2) void prefill_attn_wide(PrefillArgs
 
   const bool over = store_output<DT>(a, row, head, half, row < S, o, l);
   if constexpr (std::is_same_v<DT, BF16>)
-    if (__syncthreads_or(over)) attend<DT, kWideWaves>(a, s_tiles, g, head, q_block, over, second_pass_drop(S));
+    if (block_any(over, &s_over)) attend<DT, kWideWaves, true>(a, s_tiles, g, head, q_block, over, second_pass_drop(S));
 }
 
 constexpr int kWideBlocks = 512;
