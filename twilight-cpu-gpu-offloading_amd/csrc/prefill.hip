@@ -21,13 +21,19 @@
 // Bound: the matrix cores and, beside them, the vector unit (a score costs a
 // multiply-add, an exponential, a sum, half a conversion and half a maximum: as
 // many issue cycles as its share of the products).  8 KV heads of 4 query heads,
-// bf16: 32768 rows 8.3 ms, 1060 TFLOP/s of the causal half (library products of
-// 8192^3 and 16384^3 reach 1317 and 1587 here), against 137 ms for the score tiles in fp32 through
-// batched products, mask and softmax; 2048 rows 69 us against 1.0 ms.  The
+// bf16: 32768 rows 8.1 ms, 1090 TFLOP/s of the causal half (library products of
+// 8192^3 and 16384^3 reach 1317 and 1587 here), against 137 ms for the score tiles
+// through batched products, mask and softmax; 2048 rows 62 us against 1.0 ms.  The
 // matrix cores are busy 53% of that time, at 1.9 GHz under this load.  Two 32-row
 // query tiles a wavefront (half the LDS reads a product, one wavefront a SIMD)
 // took 10.5 ms; wavefronts 4 .. 7 a product phase behind 0 .. 3, with a barrier
 // a phase, 8.7 ms.
+//
+// The running maximum moves only when a score passes it by more than 2^8 of
+// weight, the condition that FlashAttention-4 rescales under.  What that, the fp32
+// shift of the exponents and the division at the end could get wrong at the ends of
+// the operands' range is taken care of at its place below, for 0 to 1% of the time
+// (2048 rows 61.6 -> 60.6 us in bf16, 62.5 -> 63.5 in fp16; 32768 rows 8.20 -> 8.18 ms).
 #pragma clang fp contract(off)
 
 #include <limits>
@@ -370,8 +376,11 @@ __global__ __launch_bounds__(4 * kWave, 2) void prefill_attn_kernel(PrefillArgs 
 }
 
 // Blocks of 8 wavefronts, with the three streams of neighbouring tiles
-// interleaved in each wavefront.  Against the kernel above at the same block
-// size (32768 rows of 32 heads): 17.2 M cycles and 8.9 ms, 15.8 M and 8.3 ms.
+// interleaved in each wavefront.  Against attend() with blocks of 8 (32768 rows of
+// 32 heads): 17.5 M cycles and 8.4 ms, 15.9 M and 8.1 ms.  Of the 256 registers a
+// wavefront can have, 74 spill (184 bytes a lane), none of them inside the loop over
+// the tiles: a wavefront with an odd number of tiles stores and reloads them around
+// its last.
 constexpr int kWideWaves = 8;
 constexpr int kWideThreads = kWideWaves * kWave;
 constexpr int kWideRows = kWideWaves * kQ;                      // query rows of a block
@@ -627,10 +636,12 @@ __global__ __launch_bounds__(kWideThreads, 2) void prefill_attn_wide(PrefillArgs
 constexpr int kWideBlocks = 512;
 
 // The wide kernel from two blocks a CU on; with fewer, blocks of half the rows
-// balance better, and two of them on a CU overlap by themselves.  One attention
-// layer, small against wide blocks: 2048 rows of 32 heads (256 wide blocks) 245
-// against 251 us, 4096 (512) 450 and 434, 12000 of 12 (564) 726 and 684, 8192 of
-// 32 (1024) 1145 and 1075, 32768 11.0 ms (8 wavefronts) and 10.1.
+// balance better, and two of them on a CU overlap by themselves.  The attention
+// alone, blocks of 128 rows against wide ones, bf16: 2048 rows of 32 heads (256
+// wide blocks) 62 against 73 us, 3072 (384) 100 and 104, 3584 (448) 136 and 126,
+// 4096 (512) 171 and 156, 5120 (640) 242 and 246, 8192 (1024) 587 and 546, 32768
+// 9.04 and 8.06 ms; 6000 of 16 (384) 172 and 177, 8192 of 28 (896) 521 and 491.  (At
+// 448 the wide ones are already ahead.)
 template <typename DT>
 int launch(PrefillArgs a, hipStream_t s) {
   const int heads = a.G * a.R;

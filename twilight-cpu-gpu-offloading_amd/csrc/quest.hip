@@ -347,8 +347,9 @@ __device__ void score_tile(const ScoreArgs& a, int g, int tile, uint8_t* lds) {
   const int p0 = tile * kTilePages;
   if (p0 >= a.P) return;  // block-uniform
   clear_tile_state(a, g, tile);
-  // A ragged group's length is read in the same round trip as the tile: the
-  // tile is staged up to the buffer's P pages (in bounds), and only the
+  // A ragged group's length: a launch that waits for it (waits_for_length) stages
+  // the group's own pages; a smaller one reads it in the same round trip as the
+  // tile, staged up to the buffer's P pages (in bounds).  Either way only the
   // scores of the group's own pages are written.
   // (an unconditional load: without lengths it reads the first query word
   // and ignores it)
@@ -1026,7 +1027,8 @@ int launch_score(const ScoreArgs& a, hipStream_t stream) {
   const size_t tile_bytes =
       static_cast<size_t>(2 * kTilePages) * (static_cast<size_t>(a.D) * sizeof(typename DT::storage) + 16);
   const dim3 grid(tiles * a.G);
-  // every tile row starts on 16 bytes, and the heads' accumulators fit the registers
+  // every tile row starts on 16 bytes; up to 8 heads, a wavefront each for the combine (at 8 the queries' scalars
+  // just pass the registers: score_order.h)
   const bool aligned = ((reinterpret_cast<uintptr_t>(a.pmin) | reinterpret_cast<uintptr_t>(a.pmax)) % 16) == 0 &&
                        (a.G == 1 || (a.group_stride * sizeof(typename DT::storage)) % 16 == 0);
   const bool tile_path = a.D == 128 && a.R <= 8 && aligned;

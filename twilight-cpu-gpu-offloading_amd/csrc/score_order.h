@@ -52,9 +52,12 @@ __device__ __forceinline__ void select8(const uint8_t* mn, const uint8_t* mx, co
 // d mod 32 in that range) for every head: it reads and widens each of its
 // channels' min and max once, whatever the number of heads, where a wavefront
 // per head read both rows again for each.  The queries are wave-uniform and
-// stay in scalar registers (constant address space), so the q > 0 choice is a
+// live in scalar registers (constant address space), so the q > 0 choice is a
 // scalar mask and a head costs three vector instructions a channel (select,
-// multiply, add).  The accumulators and their adjacent-pair tree are those of
+// multiply, add).  At 8 heads they are more than the registers beside the rest:
+// 22 scalars (25 of fp32 metadata, 10 there at 7 heads) wait in vector lanes, a
+// lane read each; 8 heads, 32K, still 31.0 -> 29.3 us a layer against the
+// wavefront a head.  The accumulators and their adjacent-pair tree are those of
 // the 32-accumulator order: the in-lane tree covers 4, the combine the other 8.
 constexpr int kScoreWaves = 8;
 
