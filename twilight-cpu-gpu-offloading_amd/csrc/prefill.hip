@@ -120,13 +120,15 @@ __device__ __forceinline__ float both_halves_sum(float x) {
 // A weight is 2^(x unit - shift) of a score x: unit = scale_log2 and shift =
 // m scale_log2 against the row's maximum m, one multiply-add a score.  The shift
 // is rounded, by up to half a unit in its last place for every key of the row
-// alike; past kNearShift (2^-15 there), where that would in the end be
-// hundreds of powers of two, the scores themselves become (x - m) scale_log2
-// first, 0 for the maximum.
+// alike: 2^-11 at kNearShift, no more than the scores themselves, but in the end
+// hundreds of powers of two.  Past it the scores become (x - m) scale_log2 first,
+// 0 for the maximum; the bound leaves the largest scores that fp16 holds (65504 /
+// sqrt(128), a shift of 8353) to the multiply-add.  8192 rows of 32 heads, bf16: 521
+// us with shifts up to the bound, 600 past it.
 //
 // A row whose keys so far all score -inf has no maximum yet: against 0 those keys
 // weigh 0 (-inf against -inf is a NaN that would stay in the row's sums).
-constexpr float kNearShift = 1024.0f;
+constexpr float kNearShift = 16384.0f;
 struct Exponents {
   float unit, shift;
   __device__ __forceinline__ Exponents(f32x16 (&sc)[2], float m, float scale_log2, float drop)
